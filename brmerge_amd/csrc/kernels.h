@@ -82,8 +82,7 @@ hipError_t order_tasks(const uint32_t* keys, int n, uint32_t* keys_out, int* idx
 // rmed.hip (register tier; cap = products per row, <= WMED_CAP)
 hipError_t launch_rmed_numeric(const int* rows, int n, const RowArgs& a, const OutArgs& o, hipStream_t s, int cap);
 // Exact row lengths of register-tier rows (ip <= cap, at most 64 lists) by
-// an LDS column bitmap; only for B of at most 2^20 columns (rmed_count_fits).
-bool rmed_count_fits(int N);
+// LDS column bitmaps.
 // Largest register-tier row (products) for B of N columns under the current
 // knobs: WMED_CAP_BITMAP where the bitmap ranks apply, else WMED_CAP.
 int rmed_max_cap(int N);

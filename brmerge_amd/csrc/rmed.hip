@@ -20,16 +20,12 @@
 //      keeps one pending left subtree per height;
 //   4. run heads are compacted with ballots and written to C (Precise), or
 //      to C-bar with the row length (Upper).
-//   Bitmap variants (B of at most RB2_SPAN columns, R >= 4): the columns set
-//   bits of an LDS bitmap -- flat over the row's column span in chunks of
-//   2^15 columns (B of at most RB_SPAN columns), or in two levels (level 1
-//   numbers the 64-column words in use, level 2 holds those words) -- and
-//   popcount ranks give each product its output position; products (still
-//   in registers) are bucketed by position into the ranks' LDS, and each
-//   bucket is folded in list-position order -- no sort.
+//   Bitmap variant (R >= 4): popcount ranks over LDS bitmaps in levels of
+//   64-way fan-out give each product its output position; products (still in
+//   registers) are bucketed by position into the ranks' LDS, and each bucket
+//   is folded in list-position order -- no sort.
 // The symbolic count of these rows (k_rmed_count) uses the same list lookup
-// and bitmaps; B of more than RB2_SPAN columns takes the wavefront hash
-// kernel of lds.hip.
+// and bitmaps.
 #include <limits.h>
 
 #include <algorithm>
@@ -90,43 +86,49 @@ struct RmLists {
 };
 static_assert(sizeof(RmLists) <= sizeof(RmSmem<2, uint32_t>), "list table fits the smallest variant");
 
-// Bitmap variants: the row's columns set bits of an LDS bitmap, popcount
-// ranks give every product its output position, products are bucketed by
-// position and each bucket is summed in list-position order -- O(ip) work
-// instead of a sort.  Phase A (ranks) and phase B (buckets) share the LDS;
-// the products stay in registers until phase B places them.
-//   flat (B with at most RB_SPAN columns): one bitmap over the row's column
-//     span, in chunks of RB_WORDS words (two at most);
-//   two-level (B with at most RB2_SPAN columns): level 1 has one bit per
-//     64-column word of the span, and its popcount ranks number the words
-//     in use; level 2 holds those words only (at most one per product).
-constexpr int RB_SPAN = 1 << 16;   // flat: columns of B
-constexpr int RB_WORDS = 512;      // flat: bitmap words of one chunk of the row's column span
-constexpr int RB2_SPAN = 1 << 20;  // two-level: columns of B
-constexpr int RB2_L1 = RB2_SPAN / 64 / 64;  // level-1 words
-struct RbRanks {
-    unsigned long long bm[RB_WORDS];
-    unsigned short wrank[RB_WORDS];
-};
+// Bitmap variant: popcount ranks over LDS bitmaps give every product its
+// output position, products are bucketed by position and each bucket is
+// summed in list-position order -- O(ip) work instead of a sort.
+//
+// Ranks come in levels of 64-way fan-out.  The top level has one bit per
+// 2^SH columns of the row's own column span, SH the least of 0, 6, 12, 18
+// for which the span fits RB_NW words of 64 bits; each level below holds one
+// 64-bit word per bit set above it (at most one per product), so its words
+// are numbered by the popcount ranks of the level above, and the ranks of
+// the last level (SH = 0) are the output positions.  A banded row takes one
+// level of a few words whatever N is, a row spread over 2^20 columns two,
+// over 2^26 three.  The levels share one LDS area (a level is dead once its
+// ranks are in registers), and phase B (the buckets) reuses it; the products
+// stay in registers until phase B places them.
+//
+// Measured on MI355X (kernel time, before: a flat bitmap in up to two chunks
+// or two fixed levels, one wave scan per 64 words, two atomics per product,
+// pending subtrees in registers; a 64-bit bitonic sort above 2^20 columns):
+// 1.15e6 rows of 257-512 products, N <= 65,536: 3.45 -> 3.01 ms, 1,312 -> 810
+// VALU instructions per row; 1.30e6 rows of 65-256 products, N = 1.5e6: 4.04
+// -> 1.68 ms, and their count 1.07 (hash) -> 0.82 ms.
 template <int R>
-struct Rb2Ranks {
-    unsigned long long l1[RB2_L1];
-    unsigned short l1rank[RB2_L1];
-    unsigned long long l2[64 * R];
-    unsigned short l2rank[64 * R];
+constexpr int rb_words() {
+    return R < 4 ? 256 : 64 * R;  // words of one level: at least one per product
+}
+template <int R>
+struct RbRanks {
+    unsigned w[2 * rb_words<R>()];  // 64-bit words, low half first
+    unsigned rank[rb_words<R>()];   // bits set before the low half | before the high half << 16
 };
-template <int R, bool TWO>
+// Columns of the outputs: 16 bits while B has at most RB_NARROW columns.
+constexpr int RB_NARROW = 1 << 16;
+template <int R, bool WIDE>
 struct RbBuckets {
-    double val[64 * R];    // contributions, bucket by bucket
-    unsigned cnt[32 * R];  // 16-bit bucket counters, two per word (bucket 2i low, 2i + 1 high)
-    // bucket column (two-level) or bucket column minus the span's first column (flat)
-    typename std::conditional<TWO, int, unsigned short>::type oc[64 * R];
-    unsigned char lp[64 * R];  // list position of each contribution
+    double val[64 * R];         // contributions, bucket by bucket
+    unsigned cnt[32 * R + 1];   // 16-bit bucket counters, then offsets, two per word (bucket 2i low, 2i + 1 high)
+    typename std::conditional<WIDE, int, unsigned short>::type oc[64 * R];
+    unsigned char lp[64 * R];   // list position of each contribution
 };
-template <int R, bool TWO>
+template <int R, bool WIDE>
 union RbSmem {
-    typename std::conditional<TWO, Rb2Ranks<R>, RbRanks>::type a;
-    RbBuckets<R, TWO> b;
+    RbRanks<R> a;
+    RbBuckets<R, WIDE> b;
     RmLists l;
 };
 static_assert(64 * 32 <= 0xffff, "bucket offsets in 16 bits");
@@ -136,84 +138,55 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// Inclusive scan over the wavefront with DPP moves (Hillis-Steele within
-// rows of 16 lanes, then row broadcasts): no LDS round trips.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp_add(int x) {
-    return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
-}
-__device__ __forceinline__ int wave_incl_scan_dpp(int x) {
-    x = dpp_add<0x111, 0xF>(x);  // row_shr:1
-    x = dpp_add<0x112, 0xF>(x);  // row_shr:2
-    x = dpp_add<0x114, 0xF>(x);  // row_shr:4
-    x = dpp_add<0x118, 0xF>(x);  // row_shr:8
-    x = dpp_add<0x142, 0xA>(x);  // row_bcast15 into rows 1 and 3
-    x = dpp_add<0x143, 0xC>(x);  // row_bcast31 into rows 2 and 3
-    return x;
-}
-
-// Aligned-tree fold over leaves visited in increasing list position: keeps
-// one pending left subtree per height (siblings added left + right, a node
-// with one present child passes it through).
-struct TreeFold {
-    double lv[RM_LOGL];
-    double cur;
+// Sum of one bucket (m >= 3 contributions from distinct lists) as the
+// aligned tree over list positions: one pass over the contributions in list
+// order with the pending left subtrees on a stack.  The pending heights
+// shrink towards the top of the stack, so one bit mask holds them; when the
+// next list first differs from the last one at bit d, the pending subtrees
+// below height d are complete on its left and are added (left + right), and
+// the sum waits at height d.  The stack takes the place of contributions
+// already read (LDS), which keeps a push to about a dozen instructions (with
+// the stack in registers, one slot per height, every push selects over all
+// heights).
+__device__ double rb_bucket_sum(unsigned char* lp, double* val, int m) {
+    int prev = lp[0];
+    // contributions placed by one register step of the wavefront may be out
+    // of list order: order the bucket first
+    for (int t = 1; t < m; ++t) {
+        const int l = lp[t];
+        if (l < prev) {
+            const double x = val[t];
+            int u = t;
+            for (; u > 0 && (int)lp[u - 1] > l; --u) {
+                lp[u] = lp[u - 1];
+                val[u] = val[u - 1];
+            }
+            lp[u] = (unsigned char)l;
+            val[u] = x;
+        } else {
+            prev = l;
+        }
+    }
+    prev = lp[0];
+    double cur = val[0];
     unsigned pend = 0u;
-    int prev;
-    __device__ TreeFold(int l, double v) : cur(v), prev(l) {}
-    __device__ void push(int l, double x) {
-        const int d = 31 - __clz(prev ^ l);
-        double v = cur;
-#pragma unroll
-        for (int h = 0; h < RM_LOGL; ++h)
-            if (h < d && ((pend >> h) & 1u)) v = fadd(lv[h], v);
-#pragma unroll
-        for (int h = 0; h < RM_LOGL; ++h)
-            if (h == d) lv[h] = v;
-        pend = (pend & ~((1u << d) - 1u)) | (1u << d);
+    int top = 0;
+    for (int t = 1; t < m; ++t) {
+        const int l = lp[t];
+        const double x = val[t];
+        const unsigned bit = 1u << (31 - __clz(prev ^ l));
+        unsigned low = pend & (bit - 1u);
+        pend = (pend & ~(bit - 1u)) | bit;
+        while (low) {
+            cur = fadd(val[--top], cur);
+            low &= low - 1u;
+        }
+        val[top++] = cur;
         cur = x;
         prev = l;
     }
-    __device__ double finish() const {
-        double v = cur;
-#pragma unroll
-        for (int h = 0; h < RM_LOGL; ++h)
-            if ((pend >> h) & 1u) v = fadd(lv[h], v);
-        return v;
-    }
-};
-
-// Sum of one bucket (m >= 3 contributions from distinct lists, list
-// positions lp[0..m), values val[0..m)).  Contributions placed by one
-// register step of the wavefront may be out of list order; one pass folds
-// a bucket that is in order, others visit their leaves by a search.
-__device__ double rb_bucket_sum(const unsigned char* lp, const double* val, int m) {
-    {
-        TreeFold f(lp[0], val[0]);
-        int t = 1;
-        for (; t < m; ++t) {
-            const int l = lp[t];
-            if (l < f.prev) break;
-            f.push(l, val[t]);
-        }
-        if (t == m) return f.finish();
-    }
-    unsigned long long mask = 0ull;
-    for (int t = 0; t < m; ++t) mask |= 1ull << lp[t];
-    auto leaf = [&](int l) {
-        int t = 0;
-        while (lp[t] != l) ++t;
-        return val[t];
-    };
-    int l = __ffsll((long long)mask) - 1;
-    mask &= mask - 1ull;
-    TreeFold f(l, leaf(l));
-    while (mask) {
-        l = __ffsll((long long)mask) - 1;
-        mask &= mask - 1ull;
-        f.push(l, leaf(l));
-    }
-    return f.finish();
+    while (top > 0) cur = fadd(val[--top], cur);
+    return cur;
 }
 
 // Stage 1 of a row (A entries a0 .. a0 + L, products base .. base + ip):
@@ -263,40 +236,17 @@ __device__ __forceinline__ void rm_products(const RowArgs& a, int a0, int L, int
     wave_lds_sync();  // the table is read before its area is reused
 }
 
-// Exclusive ranks of n words' popcounts into rank[0..n), consecutive lanes
-// on consecutive words, at most NI steps of 64 words; returns the total.
-template <int NI>
-__device__ __forceinline__ int rank_words(const unsigned long long* bm, unsigned short* rank, int n) {
-    const int lane = lane_id();
-    int tot = 0;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        if (i * BRM_WAVE >= n) break;  // uniform
-        const int w = i * BRM_WAVE + lane;
-        const int pc = w < n ? __popcll(bm[w]) : 0;
-        const int inc = wave_incl_scan_dpp(pc);
-        if (w < n) rank[w] = (unsigned short)(tot + inc - pc);
-        tot += __shfl(inc, BRM_WAVE - 1, BRM_WAVE);
-    }
-    return tot;
+// Bits of w below bit b (b taken mod 32).
+__device__ __forceinline__ int popc_below(unsigned w, unsigned b) {
+    return __popc(__builtin_amdgcn_ubfe(w, 0u, b & 31u));
 }
 
-// Products of product indices 64 r + lane < ip: column cl[r] & CL_COL, list
-// position cl[r] >> CL_LP, value prod[r]; B has at most RB_SPAN (flat) or
-// RB2_SPAN (two-level) columns, nw words of them.
-constexpr int CL_LP = 20;
-constexpr int CL_COL = (1 << CL_LP) - 1;
-static_assert(RB2_SPAN <= CL_COL + 1, "columns beside the list position");
-template <int R, bool TWO>
-__device__ void rmed_bitmap(const int (&cl)[R], const double (&prod)[R], int ip, int nw, int row, int64_t base,
-                            const OutArgs& o, RbSmem<R, TWO>& sh) {
+// Minimum and maximum of the products' columns over the wavefront.
+template <int R>
+__device__ __forceinline__ void col_range(const int (&col)[R], int ip, int& cmn, int& cmx) {
     const int lane = lane_id();
-    int col[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) col[r] = cl[r] & CL_COL;
-    RbBuckets<R, TWO>& B = sh.b;
-    // only the words between the row's smallest and largest column are used
-    int cmn = INT_MAX, cmx = 0;
+    cmn = INT_MAX;
+    cmx = -1;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         if (r * 64 + lane < ip) {
@@ -304,148 +254,136 @@ __device__ void rmed_bitmap(const int (&cl)[R], const double (&prod)[R], int ip,
             cmx = max(cmx, col[r]);
         }
     }
+    // prefix extremes with DPP moves; the last lane holds the wavefront's
+    auto mn = [](int x, int y) { return min(x, y); };
+    auto mx = [](int x, int y) { return max(x, y); };
+    cmn = mn(cmn, dpp_mov<0x111, 0xF>(cmn, INT_MAX));
+    cmx = mx(cmx, dpp_mov<0x111, 0xF>(cmx, -1));
+    cmn = mn(cmn, dpp_mov<0x112, 0xF>(cmn, INT_MAX));
+    cmx = mx(cmx, dpp_mov<0x112, 0xF>(cmx, -1));
+    cmn = mn(cmn, dpp_mov<0x114, 0xF>(cmn, INT_MAX));
+    cmx = mx(cmx, dpp_mov<0x114, 0xF>(cmx, -1));
+    cmn = mn(cmn, dpp_mov<0x118, 0xF>(cmn, INT_MAX));
+    cmx = mx(cmx, dpp_mov<0x118, 0xF>(cmx, -1));
+    cmn = mn(cmn, dpp_mov<0x142, 0xA>(cmn, INT_MAX));
+    cmx = mx(cmx, dpp_mov<0x142, 0xA>(cmx, -1));
+    cmn = mn(cmn, dpp_mov<0x143, 0xC>(cmn, INT_MAX));
+    cmx = mx(cmx, dpp_mov<0x143, 0xC>(cmx, -1));
+    cmn = wave_last(cmn);
+    cmx = wave_last(cmx);
+}
+
+// The top level of a row with columns in [cmn, cmx]: its shift, and the
+// words it takes.
+template <int R>
+__device__ __forceinline__ int top_level(int cmn, int cmx, int& nw) {
+    int sh = 0;
+    while (((cmx >> sh) - (cmn >> sh)) >> 6 >= rb_words<R>()) sh += 6;
+    nw = (((cmx >> sh) - (cmn >> sh)) >> 6) + 1;
+    return sh;
+}
+
+// One level: bit idx[r] of every product r * 64 + lane < ip set in nw words
+// of cleared bitmap.  Returns with the bits visible to the wavefront.
+template <int R>
+__device__ __forceinline__ void level_bits(RbRanks<R>& A, const int (&idx)[R], int ip, int nw) {
+    const int lane = lane_id();
+    unsigned long long* w64 = reinterpret_cast<unsigned long long*>(A.w);
+#pragma unroll 1
+    for (int i = 0; i < nw; i += BRM_WAVE) w64[i + lane] = 0ull;  // rb_words is a whole number of steps
+    wave_lds_sync();
 #pragma unroll
-    for (int d = BRM_WAVE / 2; d > 0; d >>= 1) {
-        cmn = min(cmn, __shfl_xor(cmn, d, BRM_WAVE));
-        cmx = max(cmx, __shfl_xor(cmx, d, BRM_WAVE));
+    for (int r = 0; r < R; ++r)
+        if (r * 64 + lane < ip) atomicOr(&A.w[idx[r] >> 5], 1u << (idx[r] & 31));
+    wave_lds_sync();
+}
+
+// Ranks of the nw words (exclusive prefix of their popcounts, one per half
+// word), two steps of 64 words per wave scan (16 bits each: a step holds at
+// most 4,096 bits); returns the number of bits set.
+template <int R>
+__device__ __forceinline__ int level_ranks(RbRanks<R>& A, int nw) {
+    const int lane = lane_id();
+    const unsigned long long* w64 = reinterpret_cast<const unsigned long long*>(A.w);
+    int tot = 0;
+#pragma unroll 1
+    for (int i = 0; i < nw; i += 2 * BRM_WAVE) {
+        const bool two = i + BRM_WAVE < nw;  // uniform
+        const unsigned long long x = w64[i + lane];
+        const unsigned long long y = two ? w64[i + BRM_WAVE + lane] : 0ull;
+        const int xl = __popc((unsigned)x), yl = __popc((unsigned)y);
+        const int xc = xl + __popc((unsigned)(x >> 32)), yc = yl + __popc((unsigned)(y >> 32));
+        const int inc = wave_incl_scan(xc | (yc << 16));
+        const int all = wave_last(inc);
+        const int ex = tot + (inc & 0xffff) - xc;
+        A.rank[i + lane] = (unsigned)(ex | ((ex + xl) << 16));
+        tot += all & 0xffff;
+        if (two) {
+            const int ey = tot + (int)((unsigned)inc >> 16) - yc;
+            A.rank[i + BRM_WAVE + lane] = (unsigned)(ey | ((ey + yl) << 16));
+            tot += (int)((unsigned)all >> 16);
+        }
     }
-    const int w0 = cmn >> 6, w1 = min((cmx >> 6) + 1, nw);
-    const int cbase = TWO ? 0 : w0 * 64;  // flat: columns of the span are cbase + [0, 2^16)
-    int nout = 0;
+    wave_lds_sync();
+    return tot;
+}
+
+// Every product's rank among the bits set: into idx.
+template <int R>
+__device__ __forceinline__ void level_lookup(const RbRanks<R>& A, int (&idx)[R], int ip) {
+    const int lane = lane_id();
+    const unsigned short* rk = reinterpret_cast<const unsigned short*>(A.rank);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (r * 64 + lane < ip) idx[r] = rk[idx[r] >> 5] + popc_below(A.w[idx[r] >> 5], (unsigned)idx[r]);
+    wave_lds_sync();  // read before the area is cleared or reused
+}
+
+// Products of product indices 64 r + lane < ip: column col[r], list position
+// lp[r], value prod[r].
+template <int R, bool WIDE>
+__device__ __forceinline__ void rmed_bitmap(const int (&col)[R], const int (&lp)[R], const double (&prod)[R], int ip,
+                                            int row, int64_t base, const OutArgs& o, RbSmem<R, WIDE>& sh) {
+    const int lane = lane_id();
     int pos[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) pos[r] = 0;
-    if constexpr (!TWO) {
-        constexpr int WPL = RB_WORDS / BRM_WAVE;  // bitmap words per lane and chunk, at most
-        RbRanks& A = sh.a;
-        // column - cbase of each product; lanes past the row hold a value no
-        // chunk takes
-        int bc[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) bc[r] = r * 64 + lane < ip ? col[r] - cbase : (1 << 30);
-        // the span in chunks of RB_WORDS words (two at most): bits, ranks and
-        // the positions of the chunk's products; ranks carry across chunks
-        auto chunk = [&](int wc) {
-            const int nwc = min(RB_WORDS, w1 - w0 - wc);
-#pragma unroll
-            for (int i = 0; i < WPL; ++i) {
-                const int w = i * BRM_WAVE + lane;
-                if (w < nwc) A.bm[w] = 0ull;
-            }
-            wave_lds_sync();
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const unsigned bit = (unsigned)(bc[r] - wc * 64);
-                if (bit < (unsigned)(RB_WORDS * 64)) atomicOr(&A.bm[bit >> 6], 1ull << (bit & 63));
-            }
-            wave_lds_sync();
-            const int base_rank = nout;
-            nout += rank_words<WPL>(A.bm, A.wrank, nwc);
-            wave_lds_sync();
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const unsigned bit = (unsigned)(bc[r] - wc * 64);
-                if (bit < (unsigned)(RB_WORDS * 64)) {
-                    const int wd = (int)(bit >> 6);
-                    pos[r] = base_rank + A.wrank[wd] + __popcll(A.bm[wd] & ((1ull << (bit & 63)) - 1ull));
-                }
-            }
-            wave_lds_sync();  // read before the next chunk clears
-        };
-        if (w1 > w0) chunk(0);
-        if (w1 - w0 > RB_WORDS) chunk(RB_WORDS);  // uniform
-    } else {
-        Rb2Ranks<R>& A = sh.a;
-        constexpr int L1PL = RB2_L1 / BRM_WAVE;  // level-1 words per lane, at most
-        const int n1 = (w1 - w0 + 63) >> 6;       // level-1 words in use
-#pragma unroll
-        for (int i = 0; i < L1PL; ++i) {
-            const int w = i * BRM_WAVE + lane;
-            if (w < n1) A.l1[w] = 0ull;
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (r * 64 + lane < ip) {
-                const int wid = (col[r] >> 6) - w0;
-                atomicOr(&A.l1[wid >> 6], 1ull << (wid & 63));
-            }
-        }
-        wave_lds_sync();
-        const int n2 = rank_words<L1PL>(A.l1, A.l1rank, n1);  // level-2 words (words in use)
-        wave_lds_sync();
-        int kk[R];  // level-2 word of each product
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            kk[r] = 0;
-            if (r * 64 + lane < ip) {
-                const int wid = (col[r] >> 6) - w0;
-                kk[r] = A.l1rank[wid >> 6] + __popcll(A.l1[wid >> 6] & ((1ull << (wid & 63)) - 1ull));
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-            const int q = i * BRM_WAVE + lane;
-            if (q < n2) A.l2[q] = 0ull;
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (r * 64 + lane < ip) atomicOr(&A.l2[kk[r]], 1ull << (col[r] & 63));
-        wave_lds_sync();
-        nout = rank_words<R>(A.l2, A.l2rank, n2);
-        wave_lds_sync();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (r * 64 + lane < ip)
-                pos[r] = A.l2rank[kk[r]] + __popcll(A.l2[kk[r]] & ((1ull << (col[r] & 63)) - 1ull));
-        }
-        wave_lds_sync();
-    }
-    // ranks are dead from here on
-    // bucket counters: 16 bits each, buckets 2i and 2i + 1 in word i
-    const int ncw = (nout + 1) >> 1;
-#pragma unroll
-    for (int i = 0; i < R / 2; ++i)
-        if (i * BRM_WAVE + lane < ncw) B.cnt[i * BRM_WAVE + lane] = 0u;
-    wave_lds_sync();
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if (r * 64 + lane < ip) {
-            atomicAdd(&B.cnt[pos[r] >> 1], 1u << ((pos[r] & 1) << 4));
-            // every writer stores the same column
-            if constexpr (TWO) B.oc[pos[r]] = col[r];
-            else B.oc[pos[r]] = (unsigned short)(col[r] - cbase);
-        }
-    }
-    wave_lds_sync();
+    int nout;
     {
-        int carry = 0;  // bucket offsets: a scan per step of 128 buckets, carried
+        int cmn, cmx, nw;
+        col_range<R>(col, ip, cmn, cmx);
+        int s = top_level<R>(cmn, cmx, nw);
+        const int top = cmn >> s;
 #pragma unroll
-        for (int i = 0; i < R / 2; ++i) {
-            if (i * BRM_WAVE >= ncw) break;  // uniform
-            const int q2 = i * BRM_WAVE + lane;
-            const unsigned w = q2 < ncw ? B.cnt[q2] : 0u;
-            const int c0 = (int)(w & 0xffffu), t = c0 + (int)(w >> 16);
-            const int inc = wave_incl_scan_dpp(t);
-            const int ex = carry + inc - t;
-            if (q2 < ncw) B.cnt[q2] = (unsigned)ex | ((unsigned)(ex + c0) << 16);
-            carry += __shfl(inc, BRM_WAVE - 1, BRM_WAVE);
+        for (int r = 0; r < R; ++r) pos[r] = (col[r] >> s) - top;
+#pragma unroll 1
+        for (;;) {  // uniform: one to four levels
+            level_bits<R>(sh.a, pos, ip, nw);
+            nout = level_ranks<R>(sh.a, nw);
+            level_lookup<R>(sh.a, pos, ip);
+            if (s == 0) break;
+            s -= 6;
+            nw = nout;
+#pragma unroll
+            for (int r = 0; r < R; ++r) pos[r] = pos[r] * 64 + ((col[r] >> s) & 63);
         }
     }
+    // ---- ranks are dead from here on: contributions per output; a
+    // product's arrival is its place in its bucket (kept above the position)
+    RbBuckets<R, WIDE>& B = sh.b;
+    const int ncw = (nout + 1) >> 1;
+#pragma unroll 1
+    for (int i = lane; i < ncw; i += BRM_WAVE) B.cnt[i] = 0u;
     wave_lds_sync();
+    int most = 0;  // largest arrival of this lane's products
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         if (r * 64 + lane < ip) {
             const unsigned sft = (unsigned)(pos[r] & 1) << 4;
-            const int slot = (int)((atomicAdd(&B.cnt[pos[r] >> 1], 1u << sft) >> sft) & 0xffffu);
-            B.val[slot] = prod[r];
-            B.lp[slot] = (unsigned char)(cl[r] >> CL_LP);
+            const int arr = (int)((atomicAdd(&B.cnt[pos[r] >> 1], 1u << sft) >> sft) & 0xffffu);
+            most = max(most, arr);
+            if (arr == 0) B.oc[pos[r]] = (typename std::conditional<WIDE, int, unsigned short>::type)col[r];
+            pos[r] |= arr << 16;
         }
     }
-    wave_lds_sync();
-    // counter q is now the end of bucket q
-    auto bend = [&](int q) { return (int)((B.cnt[q >> 1] >> ((q & 1) << 4)) & 0xffffu); };
     int* dcol;
     double* dval;
     int64_t dcap;
@@ -459,20 +397,79 @@ __device__ void rmed_bitmap(const int (&cl)[R], const double (&prod)[R], int ip,
         dval = o.cval + base;
         dcap = ip;
     }
-    for (int q = lane; q < nout; q += BRM_WAVE) {
-        const int s = q ? bend(q - 1) : 0;
-        const int m = bend(q) - s;
-        double v;
-        if (m == 1) {
-            v = B.val[s];
-        } else if (m == 2) {
-            const double x = B.val[s], y = B.val[s + 1];
-            v = B.lp[s] < B.lp[s + 1] ? fadd(x, y) : fadd(y, x);
-        } else {
-            v = rb_bucket_sum(B.lp + s, B.val + s, m);
+    const int nst = (int)min((int64_t)nout, dcap);
+    if (__ballot(most >= 2) == 0ull) {
+        // ---- at most two contributions per output: the first to arrive
+        // waits at the output's place, the second is added to it there
+        const bool pairs = __ballot(most == 1) != 0ull;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r * 64 + lane < ip && pos[r] < 0x10000) {
+                B.val[pos[r]] = prod[r];
+                if (pairs) B.lp[pos[r]] = (unsigned char)lp[r];
+            }
         }
-        if (q < dcap) {
-            dcol[q] = cbase + (int)B.oc[q];
+        wave_lds_sync();
+        if (pairs) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (r * 64 + lane < ip && pos[r] >= 0x10000) {
+                    const int q = pos[r] & 0xffff;
+                    const double x = B.val[q];
+                    B.val[q] = (int)B.lp[q] < lp[r] ? fadd(x, prod[r]) : fadd(prod[r], x);
+                }
+            }
+            wave_lds_sync();
+        }
+#pragma unroll 1
+        for (int q = lane; q < nst; q += BRM_WAVE) {
+            dcol[q] = (int)B.oc[q];
+            dval[q] = B.val[q];
+        }
+    } else {
+        // ---- bucket offsets (exclusive scan of the counters, two steps of
+        // 128 buckets per wave scan), then every product to its slot
+        wave_lds_sync();
+        int tot = 0;
+#pragma unroll 1
+        for (int i = 0; i < ncw; i += 2 * BRM_WAVE) {
+            const int p = i + lane, q = i + BRM_WAVE + lane;
+            const unsigned x = p < ncw ? B.cnt[p] : 0u, y = q < ncw ? B.cnt[q] : 0u;
+            const int x0 = (int)(x & 0xffffu), y0 = (int)(y & 0xffffu);
+            const int xt = x0 + (int)(x >> 16), yt = y0 + (int)(y >> 16);
+            const int inc = wave_incl_scan(xt | (yt << 16));
+            const int all = wave_last(inc);
+            const int ex = tot + (inc & 0xffff) - xt;
+            tot += all & 0xffff;
+            const int ey = tot + (int)((unsigned)inc >> 16) - yt;
+            tot += (int)((unsigned)all >> 16);
+            if (p < ncw) B.cnt[p] = (unsigned)(ex | ((ex + x0) << 16));
+            if (q < ncw) B.cnt[q] = (unsigned)(ey | ((ey + y0) << 16));
+        }
+        unsigned short* off = reinterpret_cast<unsigned short*>(B.cnt);
+        if (lane == 0) off[nout] = (unsigned short)ip;
+        wave_lds_sync();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (r * 64 + lane < ip) {
+                const int slot = off[pos[r] & 0xffff] + (pos[r] >> 16);
+                B.val[slot] = prod[r];
+                B.lp[slot] = (unsigned char)lp[r];
+            }
+        }
+        wave_lds_sync();
+#pragma unroll 1
+        for (int q = lane; q < nst; q += BRM_WAVE) {
+            const int s = off[q];
+            const int m = off[q + 1] - s;
+            double v = B.val[s];
+            if (m == 2) {
+                const double y = B.val[s + 1];
+                v = B.lp[s] < B.lp[s + 1] ? fadd(v, y) : fadd(y, v);
+            } else if (m > 2) {
+                v = rb_bucket_sum(B.lp + s, B.val + s, m);
+            }
+            dcol[q] = (int)B.oc[q];
             dval[q] = v;
         }
     }
@@ -525,10 +522,16 @@ __device__ __forceinline__ void wave_bitonic_sort(KT (&key)[R], int rr) {
     }
 }
 
-// MODE 0: sort; 1: flat bitmap (B of at most RB_SPAN columns); 2: two-level
-// bitmap (B of at most RB2_SPAN columns).
+// Waves per SIMD the register allocation must leave room for.
+template <int R>
+constexpr int rm_waves() {
+    return R <= 4 ? 8 : R == 8 ? 6 : R == 16 ? 4 : 2;
+}
+
+// MODE 0: sort; 1: bitmap ranks (B of at most RB_NARROW columns); 2: bitmap
+// ranks, any number of columns.
 template <int R, typename KT, int MODE>
-__global__ __launch_bounds__(BRM_WAVE) void k_rmed(const int* __restrict__ rows, int nrows, RowArgs a, OutArgs o) {
+__global__ __launch_bounds__(BRM_WAVE, rm_waves<R>()) void k_rmed(const int* __restrict__ rows, int nrows, RowArgs a, OutArgs o) {
     using Key = RmKey<R, KT>;
     // one of the layouts, sized for the variant; the list table of stage 1
     // overlays the start of each
@@ -560,10 +563,12 @@ __global__ __launch_bounds__(BRM_WAVE) void k_rmed(const int* __restrict__ rows,
 
     // ---- bitmap ranks instead of a sort
     if constexpr (MODE != 0) {
-        int cl[R];
+        // list positions stay in registers as they are: left to itself the
+        // compiler carries their derivation along (245 VGPRs instead of 120
+        // at R = 16, spills at R = 32)
 #pragma unroll
-        for (int r = 0; r < R; ++r) cl[r] = col[r] | (lp[r] << CL_LP);
-        rmed_bitmap<R, MODE == 2>(cl, prod, ip, (a.N + 63) >> 6, row, base, o, shm);
+        for (int r = 0; r < R; ++r) asm volatile("" : "+v"(lp[r]));
+        rmed_bitmap<R, MODE == 2>(col, lp, prod, ip, row, base, o, shm);
         return;
     }
     KT key[R];
@@ -654,28 +659,17 @@ __global__ __launch_bounds__(BRM_WAVE) void k_rmed(const int* __restrict__ rows,
 }
 
 // Symbolic count of register-tier rows: the row's length is the number of
-// distinct columns, the bits set in an LDS bitmap.
-//   flat (B with at most RB_SPAN columns): a bitmap of CB_BITS columns, one
-//     pass per CB_BITS of the row's column span (at most two);
-//   two-level (B with at most RB2_SPAN columns): as the numeric variant's
-//     ranks -- level 1 numbers the 64-column words in use, level 2 holds them.
-constexpr int CB_WORDS = 512;
-constexpr int CB_BITS = CB_WORDS * 64;
-template <int R, bool TWO>
+// bits set in the last level of the numeric variant's bitmaps.
+template <int R>
 union RcSmem {
     RmLists l;
-    unsigned long long bm[CB_WORDS];
-    struct {
-        unsigned long long l1[RB2_L1];
-        unsigned short l1rank[RB2_L1];
-        unsigned long long l2[TWO ? 64 * R : 1];
-    } a;
+    RbRanks<R> a;
 };
 
-template <int R, bool TWO>
+template <int R>
 __global__ __launch_bounds__(BRM_WAVE) void k_rmed_count(const int* __restrict__ rows, int nrows, RowArgs a,
                                                          int64_t* __restrict__ nnzrow) {
-    __shared__ RcSmem<R, TWO> sh;
+    __shared__ RcSmem<R> sh;
     const int lane = lane_id();
     const int row = rows[blockIdx.x];
     const int a0 = a.arpt[row];
@@ -686,82 +680,33 @@ __global__ __launch_bounds__(BRM_WAVE) void k_rmed_count(const int* __restrict__
     double sv[R];
     rm_products<R, false>(a, a0, L, base, ip, sh.l, bi, lp, sv);
     int col[R];
-    int cmn = INT_MAX, cmx = -1;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        col[r] = INT_MAX;
-        if (r * 64 + lane < ip) {
-            col[r] = a.bcol[bi[r]];
-            cmn = min(cmn, col[r]);
-            cmx = max(cmx, col[r]);
-        }
+        col[r] = 0;
+        if (r * 64 + lane < ip) col[r] = a.bcol[bi[r]];
     }
+    int cmn, cmx, nw;
+    col_range<R>(col, ip, cmn, cmx);
+    int s = top_level<R>(cmn, cmx, nw);
+    const int top = cmn >> s;
+    int idx[R];
 #pragma unroll
-    for (int d = BRM_WAVE / 2; d > 0; d >>= 1) {
-        cmn = min(cmn, __shfl_xor(cmn, d, BRM_WAVE));
-        cmx = max(cmx, __shfl_xor(cmx, d, BRM_WAVE));
+    for (int r = 0; r < R; ++r) idx[r] = (col[r] >> s) - top;
+#pragma unroll 1
+    for (;;) {  // uniform
+        level_bits<R>(sh.a, idx, ip, nw);
+        if (s == 0) break;
+        nw = level_ranks<R>(sh.a, nw);
+        level_lookup<R>(sh.a, idx, ip);
+        s -= 6;
+#pragma unroll
+        for (int r = 0; r < R; ++r) idx[r] = idx[r] * 64 + ((col[r] >> s) & 63);
     }
     int cnt = 0;
-    if constexpr (!TWO) {
-        // columns < RB_SPAN: c0 stays far from overflow; no products, no pass
-        for (int c0 = cmn & ~63; c0 <= cmx; c0 += CB_BITS) {  // uniform
-            const int nwd = min(CB_WORDS, ((cmx - c0) >> 6) + 1);
-#pragma unroll
-            for (int i = 0; i < CB_WORDS / BRM_WAVE; ++i)
-                if (i * BRM_WAVE + lane < nwd) sh.bm[i * BRM_WAVE + lane] = 0ull;
-            wave_lds_sync();
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const unsigned d = (unsigned)(col[r] - c0);
-                if (d < (unsigned)CB_BITS) atomicOr(&sh.bm[d >> 6], 1ull << (d & 63));
-            }
-            wave_lds_sync();
-#pragma unroll
-            for (int i = 0; i < CB_WORDS / BRM_WAVE; ++i)
-                if (i * BRM_WAVE + lane < nwd) cnt += __popcll(sh.bm[i * BRM_WAVE + lane]);
-            wave_lds_sync();  // counted before the next pass clears
-        }
-    } else if (cmx >= 0) {  // uniform: the row has products
-        constexpr int L1PL = RB2_L1 / BRM_WAVE;
-        const int w0 = cmn >> 6;
-        const int n1 = ((cmx >> 6) - w0 + 64) >> 6;  // level-1 words in use
-#pragma unroll
-        for (int i = 0; i < L1PL; ++i)
-            if (i * BRM_WAVE + lane < n1) sh.a.l1[i * BRM_WAVE + lane] = 0ull;
-        wave_lds_sync();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (r * 64 + lane < ip) {
-                const int wid = (col[r] >> 6) - w0;
-                atomicOr(&sh.a.l1[wid >> 6], 1ull << (wid & 63));
-            }
-        }
-        wave_lds_sync();
-        const int n2 = rank_words<L1PL>(sh.a.l1, sh.a.l1rank, n1);
-        wave_lds_sync();
-        int kk[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            kk[r] = 0;
-            if (r * 64 + lane < ip) {
-                const int wid = (col[r] >> 6) - w0;
-                kk[r] = sh.a.l1rank[wid >> 6] + __popcll(sh.a.l1[wid >> 6] & ((1ull << (wid & 63)) - 1ull));
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-            if (i * BRM_WAVE + lane < n2) sh.a.l2[i * BRM_WAVE + lane] = 0ull;
-        wave_lds_sync();
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (r * 64 + lane < ip) atomicOr(&sh.a.l2[kk[r]], 1ull << (col[r] & 63));
-        wave_lds_sync();
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-            if (i * BRM_WAVE + lane < n2) cnt += __popcll(sh.a.l2[i * BRM_WAVE + lane]);
-    }
-#pragma unroll
-    for (int d = BRM_WAVE / 2; d > 0; d >>= 1) cnt += __shfl_xor(cnt, d, BRM_WAVE);
+    const unsigned long long* w64 = reinterpret_cast<const unsigned long long*>(sh.a.w);
+#pragma unroll 1
+    for (int i = 0; i < nw; i += BRM_WAVE) cnt += __popcll(w64[i + lane]);
+    cnt = wave_sum(cnt);
     if (lane == 0) nnzrow[row] = cnt;
 }
 
@@ -770,8 +715,7 @@ hipError_t rmed_count_t(const int* rows, int n, const RowArgs& a, int64_t* nnzro
     const int64_t ch = launch_chunk(BRM_WAVE);
     for (int64_t b = 0; b < n; b += ch) {
         const int c = (int)std::min<int64_t>(ch, n - b);
-        if (a.N <= RB_SPAN) k_rmed_count<R, false><<<c, BRM_WAVE, 0, s>>>(rows + b, c, a, nnzrow);
-        else k_rmed_count<R, true><<<c, BRM_WAVE, 0, s>>>(rows + b, c, a, nnzrow);
+        k_rmed_count<R><<<c, BRM_WAVE, 0, s>>>(rows + b, c, a, nnzrow);
     }
     return hipGetLastError();
 }
@@ -780,11 +724,8 @@ template <int R>
 hipError_t rmed_t(const int* rows, int n, const RowArgs& a, const OutArgs& o, hipStream_t s) {
     const int64_t ch = launch_chunk(BRM_WAVE);
     const bool narrow = a.N <= 0 || (int64_t)a.N - 1 <= RmKey<R, uint32_t>::COL_MAX;
-    // the bitmap variants pay for their larger LDS footprint on rows of more
-    // than 128 products
-    const bool bm_on = R >= 4 && params().wmed_bitmap == 1;
-    const int mode = !bm_on ? 0 : a.N <= RB_SPAN ? 1 : a.N <= RB2_SPAN ? 2 : 0;
-    // rows of more than 1024 products are binned only where a bitmap variant runs
+    const int mode = params().wmed_bitmap != 1 || R < 4 ? 0 : a.N <= RB_NARROW ? 1 : 2;
+    // rows of more than 1024 products are binned only where the ranks run
     if (R > 16 && mode == 0) return hipErrorInvalidValue;
     for (int64_t b = 0; b < n; b += ch) {
         const int c = (int)std::min<int64_t>(ch, n - b);
@@ -808,26 +749,25 @@ hipError_t rmed_t(const int* rows, int n, const RowArgs& a, const OutArgs& o, hi
 
 }  // namespace
 
+// B of at most RM_WIDE columns: rows of up to WMED_CAP_BITMAP products.
+constexpr int RM_WIDE = 1 << 20;
+
 int rmed_auto_cap(int N) {
-    // The bitmap variants take rows of up to WMED_CAP_BITMAP products while
-    // B has at most RB2_SPAN columns (rows of 1025-2048 products: 2,048
-    // products per wavefront ran faster than the workgroup LDS tier).
-    // Otherwise 1024-product rows sort 32-bit keys only while N fits beside
-    // 16 bits of position and index; with 64-bit keys they run slower than
-    // the workgroup LDS tier, so the register tier then stops at 512 products.
-    if (params().wmed_bitmap == 1 && N <= RB2_SPAN) return WMED_CAP_BITMAP;
+    // With bitmap ranks rows of up to WMED_CAP_BITMAP products while B has at
+    // most RM_WIDE columns (rows of 1025-2048 products: 2,048 products per
+    // wavefront ran faster than the workgroup LDS tier).  Otherwise 1024
+    // products while 32-bit sort keys hold N columns beside 16 bits of
+    // position and index, else 512.
+    if (params().wmed_bitmap == 1 && N <= RM_WIDE) return WMED_CAP_BITMAP;
     return (int64_t)N - 1 <= RmKey<16, uint32_t>::COL_MAX ? 1024 : 512;
 }
 
 int rmed_max_cap(int N) {
-    return params().wmed_bitmap == 1 && N <= RB2_SPAN ? WMED_CAP_BITMAP : WMED_CAP;
+    return params().wmed_bitmap == 1 && N <= RM_WIDE ? WMED_CAP_BITMAP : WMED_CAP;
 }
-
-bool rmed_count_fits(int N) { return N <= RB2_SPAN; }
 
 hipError_t launch_rmed_count(const int* rows, int n, const RowArgs& a, int64_t* nnzrow, hipStream_t s, int cap) {
     if (n <= 0) return hipSuccess;
-    if (!rmed_count_fits(a.N)) return hipErrorInvalidValue;
     ProfScope ps_("k_rmed_count", s);
     if (cap <= 128) return rmed_count_t<2>(rows, n, a, nnzrow, s);
     if (cap <= 256) return rmed_count_t<4>(rows, n, a, nnzrow, s);

@@ -178,11 +178,10 @@ int brm_flop_count_dev(const int *arpt, const int *acol, int64_t nnzA, const int
  * 0 (or a driver without address reservation): into chunks copied into C.
  * small_fused (1, the default): products whose rows are all short run in
  * the three-launch fused path.  wmed_count (1, the default): the
- * wavefront tier's row lengths are counted with a column bitmap when B has
- * at most 2^20 columns; 0: with the hash count.  wmed_bitmap (1, the
- * default): the register tier ranks rows of more than 128 products with a
- * column bitmap when B has at most 2^20 columns (and then takes rows of up
- * to 2,048 products); 0: with a sort. */
+ * wavefront tier's row lengths are counted with column bitmaps; 0: with the
+ * hash count.  wmed_bitmap (1, the default): the register tier ranks rows of
+ * more than 128 products with column bitmaps (and takes rows of up to 2,048
+ * products when B has at most 2^20 columns); 0: with a sort. */
 int brm_set_param(const char *name, int64_t value);
 int64_t brm_get_param(const char *name);
 
