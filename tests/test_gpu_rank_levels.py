@@ -82,3 +82,27 @@ def test_rank_level_edges(gpu, cap, ncols, shape):
             assert_csr_equal(f(Ah, Bh), R)
     finally:
         bm.set_param("wmed_cap", old)
+
+
+@pytest.mark.parametrize("dmin,dmax", [(9, 14), (17, 22)], ids=["to_256", "to_512"])
+@pytest.mark.parametrize("rows", [16383, 32769, 140011])
+def test_several_rows_per_wavefront(gpu, rows, dmin, dmax):
+    """Row lists long enough for one, two and eight rows per wavefront (and
+    last wavefronts and shares of the XCDs that are not full), banded rows with
+    empty lists among them."""
+    bm = gpu
+    rng = np.random.default_rng(rows + dmin)
+
+    def banded(lo, hi, empty):
+        deg = rng.integers(lo, hi + 1, rows)
+        deg[rng.random(rows) < empty] = 0
+        r = np.repeat(np.arange(rows), deg)
+        key = np.unique(r * rows + np.clip(r + rng.integers(-40, 41, len(r)), 0, rows - 1))
+        rpt = np.concatenate([[0], np.cumsum(np.bincount(key // rows, minlength=rows))]).astype(np.int32)
+        return rpt, (key % rows).astype(np.int32), rng.uniform(-1, 1, len(key)), rows
+
+    A, B = banded(dmin, dmax, 0.0), banded(dmin, dmax, 0.1)
+    R = oracle.brmerge_precise(A, B, nthreads=8)
+    Ah, Bh = csr_from_tuple(A), csr_from_tuple(B)
+    for f in (bm.brmerge_precise, bm.brmerge_upper):
+        assert_csr_equal(f(Ah, Bh), R)
