@@ -89,7 +89,7 @@ def kernel_bytes(name, A, L, ip, nnz_row, tier):
     workspace passes) is never counted: it is overhead, reported apart."""
     sel = {"k_short_numeric": 1, "k_short_count": 1, "k_medium": 2, "k_sym_hash": 2, "k_sym_bitmap": 3,
            "k_medium_w": 4, "k_rmed": 4, "k_sym_hash_w": 4,
-           "k_bgroup": 3, "k_group": 3, "k_leaf": 3}
+           "k_btile": 3, "k_bgroup": 3, "k_group": 3, "k_leaf": 3}
     if name == "k_small":  # the fused short-row path finishes every row
         return 20 * int(L.sum()) + 12 * int(ip.sum()) + 12 * int(nnz_row.sum()) + 12 * len(L)
     if name not in sel:
@@ -108,7 +108,7 @@ def engine_bytes(name, st):
     workspace traffic of the intermediate tree levels."""
     if name == "k_leaf":
         return 12 * st["leaf_ip"] + 12 * st["leaf_out"] + 20 * st["leaf_tasks"]
-    if name in ("k_group", "k_bgroup"):
+    if name in ("k_group", "k_bgroup", "k_btile"):
         return 12 * st["group_in"] + 12 * st["group_out"] + 48 * st["group_tasks"]
     return None
 

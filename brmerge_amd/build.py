@@ -20,7 +20,7 @@ XCHECK = os.path.join(HERE, "libbrm_xcheck.so")
 COMPAT_CALLER = os.path.join(os.path.dirname(HERE), "tests", "compat", "compat_caller")
 
 HIP_SOURCES = ["alloc.hip", "scan.hip", "flop.hip", "short.hip", "lds.hip", "long.hip", "assemble.hip", "api.hip",
-               "batch.hip", "serve.hip", "bmerge.hip", "rmed.hip",
+               "batch.hip", "serve.hip", "bmerge.hip", "btile.hip", "rmed.hip",
                "transpose.hip", "hash.hip", "noalloc.hip", "small.hip"]
 CXX_SOURCES = ["gen.cpp"]
 

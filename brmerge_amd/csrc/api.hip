@@ -31,7 +31,7 @@
 namespace brm {
 
 Params& params() {
-    static Params p{0, MED_CAP, 0, MED_CAP, 0, 0, GROUP_CFG_BITMAP, -1, 0, 1, 0, (int64_t)1 << 30, 0, 1, 1, 1, 1};
+    static Params p{0, MED_CAP, 0, MED_CAP, 0, 0, GROUP_CFG_BITMAP, -1, 0, 1, 0, (int64_t)1 << 30, 0, 1, 1, 1, 1, 1};
     return p;
 }
 
@@ -302,6 +302,8 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
     int64_t budget = params().ws_budget_bytes;
     if (budget <= 0) budget = thread_ws_budget();
     const int64_t arena = arena_remaining();
+    const int group_cfg = params().group_cfg;
+    const bool bitmap = group_cfg == GROUP_CFG_BITMAP;
     if (arena >= 0) {
         // the arena bounds everything this function allocates: per long row,
         // 28 bytes of wave tables beside row_bytes(), and alignment slack
@@ -325,8 +327,27 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         if (last > 0 && last <= avail / 10 * 8 && last <= (int64_t)tot / 2) budget = last;
         last = budget;
     }
-    const int group_cfg = params().group_cfg;
-    const bool bitmap = group_cfg == GROUP_CFG_BITMAP;
+    // The column-tile engine where its tables pay: block boundaries and B's
+    // table rows, at most a quarter of the budget and taken off it.  Not in
+    // the fixed-buffer arena; and where they cannot be allocated the engine
+    // without tables runs.
+    Scratch tile_sc;
+    int nb = 0;
+    int *tile_cb = nullptr, *tile_brow = nullptr;
+    if (bitmap && arena < 0 && params().long_tiles) {
+        int64_t lip = 0;
+        for (int k = 0; k < nlong; ++k) lip += ip[k];
+        nb = params().long_tiles > 1 ? params().long_tiles  // that many blocks
+                                     : tile_blocks(std::min(lip, budget / 2), a.K, a.N);
+        const int64_t brow = (int64_t)a.K * (nb + 1);
+        if (nb > 0 && (tile_sc.alloc(&tile_cb, nb + 1, "column blocks") != BRM_OK ||
+                       tile_sc.alloc(&tile_brow, brow, "B block table") != BRM_OK))
+            nb = 0;
+        if (nb > 0) {
+            HIPC(launch_tile_tables(a, nb, tile_cb, tile_brow, s));
+            budget -= 4 * brow;
+        }
+    }
     const int pass_bits = bitmap ? BPASS_BITS : PASS_BITS;
     // Workspace elements row k stores in buffer b.  Pass j writes its nodes
     // below the root into buffer j & 1 and the root writes C, so with the
@@ -342,24 +363,31 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         const int J = H == 0 ? 1 : (H + pass_bits - 1) / pass_bits;
         return (b == 1 ? J >= 2 : J >= 3) ? ip[k] : 0;
     };
+    // nodes of row k below its root: rows of the node table
+    auto n_nodes = [&](int k) -> int64_t {
+        int64_t n = 0;
+        if (nb > 0)
+            for (int h = pass_bits; h < hk[k]; h += pass_bits) n += ((len[k] - 1) >> h) + 1;
+        return n;
+    };
     std::vector<int64_t> rbytes(nlong);
     for (int k = 0; k < nlong; ++k)
-        rbytes[k] = 12 * (ws_need(k, 0) + ws_need(k, 1)) + 8 * ((int64_t)2 << hk[k]) +
+        rbytes[k] = 4 * (int64_t)(nb + 1) * n_nodes(k) + 12 * (ws_need(k, 0) + ws_need(k, 1)) + 8 * ((int64_t)2 << hk[k]) +
                     (int64_t)(sizeof(GroupTask) + sizeof(LeafTask) + 2 * sizeof(Child)) * (len[k] + 16);
 
     tr.mark("long info read back");
     // ---- partition into waves and size every buffer for the largest wave
     struct Wave {
         int k0, k1;
-        int64_t ws_tot[2], sl_tot, leaf_cap, child_cap;
-        std::vector<int64_t> wsb, slb, seg;  // wsb: two per row (buffers 0 and 1)
+        int64_t ws_tot[2], sl_tot, tab_tot, leaf_cap, child_cap;
+        std::vector<int64_t> wsb, slb, tabb, seg;  // wsb: two per row (buffers 0 and 1)
     };
     std::vector<Wave> waves;
-    int64_t mx_ws[2] = {0, 0}, mx_sl = 0, mx_leaf = 0, mx_child = 0, mx_task = 0;
+    int64_t mx_ws[2] = {0, 0}, mx_sl = 0, mx_leaf = 0, mx_child = 0, mx_task = 0, mx_tab = 0;
     int mx_rows = 0;
   for (;;) {  // (the arena case re-plans with a smaller budget until the buffers fit)
     waves.clear();
-    mx_ws[0] = mx_ws[1] = mx_sl = mx_leaf = mx_child = mx_task = 0;
+    mx_ws[0] = mx_ws[1] = mx_sl = mx_leaf = mx_child = mx_task = mx_tab = 0;
     mx_rows = 0;
     for (int k0 = 0; k0 < nlong;) {
         int k1 = k0;
@@ -368,9 +396,10 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         Wave w;
         w.k0 = k0;
         w.k1 = k1;
-        w.ws_tot[0] = w.ws_tot[1] = w.sl_tot = w.leaf_cap = w.child_cap = 0;
+        w.ws_tot[0] = w.ws_tot[1] = w.sl_tot = w.tab_tot = w.leaf_cap = w.child_cap = 0;
         w.wsb.resize(2 * (size_t)(k1 - k0));
         w.slb.resize(k1 - k0);
+        w.tabb.resize(k1 - k0);
         std::vector<int64_t> capP(MAX_PASSES + 1, 0);
         for (int k = 0; k < k1 - k0; ++k) {
             const int Lr = len[k0 + k];
@@ -383,6 +412,8 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
             w.wsb[2 * k] = w.ws_tot[0];
             w.wsb[2 * k + 1] = w.ws_tot[1];
             w.slb[k] = w.sl_tot;
+            w.tabb[k] = w.tab_tot;
+            w.tab_tot += n_nodes(k0 + k);
             w.ws_tot[0] += ws_need(k0 + k, 0);
             w.ws_tot[1] += ws_need(k0 + k, 1);
             w.sl_tot += (int64_t)2 << H;
@@ -398,6 +429,7 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         mx_leaf = std::max(mx_leaf, w.leaf_cap);
         mx_child = std::max(mx_child, w.child_cap);
         mx_task = std::max(mx_task, w.seg[MAX_PASSES + 1]);
+        mx_tab = std::max(mx_tab, w.tab_tot);
         mx_rows = std::max(mx_rows, k1 - k0);
         waves.push_back(std::move(w));
         k0 = k1;
@@ -432,6 +464,7 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         mx_leaf = round_geo(mx_leaf, (int64_t)1 << 14);
         mx_child = round_geo(mx_child, (int64_t)1 << 14);
         mx_task = round_geo(mx_task, (int64_t)1 << 14);
+        mx_tab = nb > 0 ? round_geo(mx_tab * (nb + 1), (int64_t)1 << 16) : 0;  // table entries from here on
         mx_rows = (int)round_geo(mx_rows, (int64_t)1 << 10);
     }
     Scratch wsc;
@@ -449,9 +482,10 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
     // not hold the sort's buffers).
     struct WaveTables {
         int* rows_w = nullptr;
-        int64_t *wsb_d = nullptr, *slb_d = nullptr, *seg_d = nullptr, *slots = nullptr, *counters = nullptr;
+        int64_t *wsb_d = nullptr, *slb_d = nullptr, *tabb_d = nullptr, *seg_d = nullptr, *slots = nullptr, *counters = nullptr;
         GroupTask* tasks = nullptr;
         Child* children = nullptr;
+        int* node_tab = nullptr;
         uint32_t *tkey = nullptr, *tkey_out = nullptr;
         int *tidx_in = nullptr, *tidx_out = nullptr;
         unsigned char* ttmp = nullptr;
@@ -471,6 +505,10 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         BRMC(wsc.alloc(&t.rows_w, mx_rows, "wave rows"));
         BRMC(wsc.alloc(&t.wsb_d, 2 * (int64_t)mx_rows, "wave ws_base"));
         BRMC(wsc.alloc(&t.slb_d, mx_rows, "wave slot_base"));
+        if (nb > 0) {
+            BRMC(wsc.alloc(&t.tabb_d, mx_rows, "wave tab_base"));
+            BRMC(wsc.alloc(&t.node_tab, mx_tab, "node block table"));
+        }
         BRMC(wsc.alloc(&t.seg_d, MAX_PASSES + 2, "task segments"));
         BRMC(wsc.alloc(&t.slots, mx_sl, "length slots"));
         BRMC(wsc.alloc(&t.counters, CNT_N, "planner counters"));
@@ -554,6 +592,8 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         HIPC(hipMemcpyAsync(t.rows_w, rows.data() + w.k0, sizeof(int) * nw, hipMemcpyHostToDevice, ws));
         HIPC(hipMemcpyAsync(t.wsb_d, w.wsb.data(), sizeof(int64_t) * 2 * nw, hipMemcpyHostToDevice, ws));
         HIPC(hipMemcpyAsync(t.slb_d, w.slb.data(), sizeof(int64_t) * nw, hipMemcpyHostToDevice, ws));
+        if (nb > 0)
+            HIPC(hipMemcpyAsync(t.tabb_d, w.tabb.data(), sizeof(int64_t) * nw, hipMemcpyHostToDevice, ws));
         HIPC(hipMemcpyAsync(t.seg_d, w.seg.data(), sizeof(int64_t) * (MAX_PASSES + 2), hipMemcpyHostToDevice, ws));
         HIPC(launch_fill_i64(t.counters, CNT_N, 0, ws));
         HIPC(launch_fill_i64(t.slots, w.sl_tot, 0, ws));
@@ -563,6 +603,7 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         la.nrows = nw;
         la.ws_base = t.wsb_d;
         la.slot_base = t.slb_d;
+        la.tab_base = t.tabb_d;
         la.arpt = a.arpt;
         la.acol = a.acol;
         la.aval = a.aval;
@@ -611,8 +652,13 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
                                  ttmp_bytes, ws));
                 order = t.tidx_out;
             }
-            HIPC(launch_group(t.tasks + w.seg[j], cnt[CNT_TASK0 + j], t.children, a, wcol, wval, t.slots, t.counters, o,
-                              ws, group_cfg, order));
+            if (nb > 0)
+                HIPC(launch_btile(t.tasks + w.seg[j], cnt[CNT_TASK0 + j], t.children, a,
+                                  TileTabs{tile_cb, nb, tile_brow, t.node_tab}, wcol, wval, t.slots, t.counters, o,
+                                  ws, order));
+            else
+                HIPC(launch_group(t.tasks + w.seg[j], cnt[CNT_TASK0 + j], t.children, a, wcol, wval, t.slots,
+                                  t.counters, o, ws, group_cfg, order));
             ntask += cnt[CNT_TASK0 + j];
             tr.mark("group pass", cnt[CNT_TASK0 + j]);
             if (overlap && j == b1_last) HIPC(hipEventRecord(hand[par].b1_free, ws));
@@ -1621,6 +1667,10 @@ int brm_set_param(const char* name, int64_t value) {
     else if (!strcmp(name, "small_fused")) { p.small_fused = value ? 1 : 0; }
     else if (!strcmp(name, "wmed_count")) { p.wmed_count = value ? 1 : 0; }
     else if (!strcmp(name, "wmed_bitmap")) { p.wmed_bitmap = value ? 1 : 0; }
+    else if (!strcmp(name, "long_tiles")) {
+        if (value < 0 || value > 4096) return BRM_E_INVALID;
+        p.long_tiles = (int)value;
+    }
     else if (!strcmp(name, "hash_cap")) { if (value < 0 || value > HASH_CAP) return BRM_E_INVALID; p.hash_cap = (int)value; }
     else if (!strcmp(name, "sym_chunk_products")) { if (value < 1 || value > ((int64_t)1 << 30)) return BRM_E_INVALID; p.sym_chunk_products = value; }
     else return BRM_E_INVALID;
@@ -1647,6 +1697,7 @@ int64_t brm_get_param(const char* name) {
     if (!strcmp(name, "small_fused")) return p.small_fused;
     if (!strcmp(name, "wmed_count")) return p.wmed_count;
     if (!strcmp(name, "wmed_bitmap")) return p.wmed_bitmap;
+    if (!strcmp(name, "long_tiles")) return p.long_tiles;
     return -1;
 }
 

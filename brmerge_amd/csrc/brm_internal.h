@@ -87,7 +87,7 @@ struct Src {
 struct Child {
     Src src;
     int lid;
-    int pad;
+    int tab;  // table row (column-tile engine): the B row, or the node's row of the wave's node table
 };
 
 // One node above the frontier, merged from its children in one pass.
@@ -99,6 +99,7 @@ struct GroupTask {
     int64_t cbase;    // first child in the child array
     int64_t dst_off;  // element offset in destination
     int64_t slot;     // workspace: length slot of this node
+    int64_t tab;      // workspace: row of the wave's node table (column-tile engine)
 };
 
 struct LeafTask {
@@ -130,6 +131,7 @@ struct LongArgs {
     int nrows;
     const int64_t* ws_base;  // per row: [2] element offsets into workspace buffers 0 and 1
     const int64_t* slot_base;
+    const int64_t* tab_base;  // per row: its first row of the node table, or nullptr
     const int* arpt;
     const int* acol;
     const double* aval;
@@ -200,6 +202,7 @@ struct Params {
     int small_fused;           // products of few short rows in three launches (1) or the general pipeline (0)
     int wmed_count;            // wavefront tier symbolic: 1 column bitmaps, 0 hash
     int wmed_bitmap;           // register tier numeric: 1 bitmap ranks (rows > 128 products), 0 sort
+    int long_tiles;            // long rows: 1 the column-tile engine where its tables pay, 0 never, n >= 2 n blocks
 };
 
 // Shapes of the LDS tree-merge kernels, selectable at run time.

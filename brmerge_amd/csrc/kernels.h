@@ -116,6 +116,23 @@ hipError_t launch_hash_numeric(const int* rows, int n, const RowArgs& a, const O
 // lds.hip: exact row counts of hash-tier rows
 hipError_t launch_hash_count(const int* rows, int n, const RowArgs& a, int64_t* nnzrow, hipStream_t s, int cap);
 
+// btile.hip: the column-tile engine for the same tasks, planned with tab_base.
+// cb: block boundaries [nb + 1]; brow: table rows of B; node: those of the
+// wave's nodes (nb + 1 entries each)
+struct TileTabs {
+    const int* cb;
+    int nb;
+    const int* brow;
+    int* node;
+};
+// Blocks for long rows of long_ip products in all and B of K rows and N
+// columns (0: the tables do not pay).
+int tile_blocks(int64_t long_ip, int K, int N);
+hipError_t launch_tile_tables(const RowArgs& a, int nb, int* cb, int* brow, hipStream_t s);
+hipError_t launch_btile(const GroupTask* tasks, int64_t n, const Child* children, const RowArgs& a,
+                        const TileTabs& tt, int* const ws_col[2], double* const ws_val[2], int64_t* slots,
+                        int64_t* counters, const OutArgs& o, hipStream_t s, const int* order);
+
 // bmerge.hip
 hipError_t launch_bgroup(const GroupTask* tasks, int64_t n, const Child* children, const RowArgs& a,
                          int* const ws_col[2], double* const ws_val[2], int64_t* slots, int64_t* counters,

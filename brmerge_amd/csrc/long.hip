@@ -52,6 +52,13 @@ struct WsBase {
     __device__ int64_t at(int buf) const { return buf ? b1 : b0; }
 };
 
+// Row of the wave's node table that holds pass-j node (s, h_j) of a row of L
+// lists: the row's nodes of passes 1, 2, ... below the root in turn.
+__device__ __forceinline__ int64_t node_tab(int64_t base, int L, int H, int pb, int j, int s) {
+    for (int i = 1; i < j; ++i) base += ((L - 1) >> pass_height(i, H, pb)) + 1;
+    return base + (s >> pass_height(j, H, pb));
+}
+
 struct NodeK {
     int kind;
     int q;
@@ -142,7 +149,7 @@ __device__ void emit_group(const LongArgs& la, int row, int a0, const int64_t* i
             // every child starts on a multiple of 2^hprev: dropping those
             // low bits keeps the pairing and skips levels with no pairs
             c.lid = (q - s) >> hprev;
-            c.pad = 0;
+            c.tab = 0;
             la.children[cb + k] = c;
             k++;
         }
@@ -157,11 +164,13 @@ __device__ void emit_group(const LongArgs& la, int row, int a0, const int64_t* i
         T.dst_buf = 0;
         T.dst_off = final_off;
         T.slot = -1;
+        T.tab = -1;
     } else {
         T.final_dst = 0;
         T.dst_buf = j & 1;
         T.dst_off = wsb.at(j & 1) + (ipr[s] - ipr[0]);
         T.slot = slb + heap_idx(H, s, hj);
+        T.tab = -1;
     }
     const unsigned long long idx = atomicAdd((unsigned long long*)&la.counters[CNT_TASK0 + j], 1ull);
     if ((int64_t)idx >= la.task_seg[j + 1] - la.task_seg[j]) {
@@ -180,7 +189,7 @@ __device__ void emit_group(const LongArgs& la, int row, int a0, const int64_t* i
 // PL_NT / F nodes per step, one child slot per thread, with one scan and one
 // reservation of child entries for all of them.
 __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int64_t* ipr, int L, int H, int J,
-                                 WsBase wsb, int64_t slb, int64_t final_off, int* err) {
+                                 WsBase wsb, int64_t slb, int64_t tabb, int64_t final_off, int* err) {
     __shared__ int64_t sm[PL_NT / BRM_WAVE + 1];
     __shared__ int64_t cbase;
     __shared__ int64_t lead[PL_NT + 1];  // child prefix at each node's first slot; [G]: the step's total
@@ -227,7 +236,10 @@ __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int6
                     Child ch;
                     ch.src = src;
                     ch.lid = c;  // (q - s) >> hp
-                    ch.pad = 0;
+                    // the B row of a list, the table row of a node
+                    ch.tab = src.kind == SRC_VIRTUAL ? la.acol[a0 + upper_idx(ipr, q, node_end(L, q, hp), ipr[q])]
+                             : tabb >= 0            ? (int)node_tab(tabb, L, H, pb, j - 1, q)
+                                                    : 0;
                     la.children[cb + rank] = ch;
                 }
                 if (c == 0 && live) {
@@ -240,11 +252,13 @@ __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int6
                         T.dst_buf = 0;
                         T.dst_off = final_off;
                         T.slot = -1;
+                        T.tab = -1;
                     } else {
                         T.final_dst = 0;
                         T.dst_buf = j & 1;
                         T.dst_off = wsb.at(j & 1) + (ipr[s] - ipr[0]);
                         T.slot = slb + heap_idx(H, s, hj);
+                        T.tab = tabb >= 0 ? node_tab(tabb, L, H, pb, j, s) : -1;
                     }
                     const unsigned long long idx =
                         atomicAdd((unsigned long long*)&la.counters[CNT_TASK0 + j], 1ull);
@@ -277,7 +291,7 @@ __global__ __launch_bounds__(PL_NT) void k_plan(LongArgs la, int r0, int* err) {
     const int64_t slb = la.slot_base[r];
     const int64_t final_off = la.final_off ? la.final_off[row] : ipr[0];
     if (la.frontier_cap == 0 && (1 << pb) <= PL_NT) {
-        plan_no_frontier(la, row, a0, ipr, L, H, J, wsb, slb, final_off, err);
+        plan_no_frontier(la, row, a0, ipr, L, H, J, wsb, slb, la.tab_base ? la.tab_base[r] : -1, final_off, err);
         if (threadIdx.x == 0) atomicMax((unsigned long long*)&la.counters[CNT_MAXP], (unsigned long long)J);
         return;
     }

@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "brm_device.h"
+#include "bucket_sum.h"
 #include "kernels.h"
 
 namespace brm {
@@ -131,7 +132,7 @@ struct RbBuckets {
     };
     unsigned short off[64 * R + 2];  // bucket offsets
     typename std::conditional<WIDE, int, unsigned short>::type oc[64 * R];  // output columns
-    unsigned char lp[64 * R];    // list position of each contribution
+    unsigned char lp[64 * R + 8];  // list position of each contribution (read 8 at a time)
 };
 template <int R, bool WIDE>
 union RbSmem {
@@ -140,62 +141,6 @@ union RbSmem {
     RmLists l;
 };
 static_assert(64 * 32 <= 0xffff, "bucket offsets in 16 bits");
-
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// Sum of one bucket (m >= 3 contributions from distinct lists) as the
-// aligned tree over list positions: one pass over the contributions in list
-// order with the pending left subtrees on a stack.  The pending heights
-// shrink towards the top of the stack, so one bit mask holds them; when the
-// next list first differs from the last one at bit d, the pending subtrees
-// below height d are complete on its left and are added (left + right), and
-// the sum waits at height d.  The stack takes the place of contributions
-// already read (LDS), which keeps a push to about a dozen instructions (with
-// the stack in registers, one slot per height, every push selects over all
-// heights).
-__device__ double rb_bucket_sum(unsigned char* lp, double* val, int m) {
-    int prev = lp[0];
-    // contributions placed by one register step of the wavefront may be out
-    // of list order: order the bucket first
-    for (int t = 1; t < m; ++t) {
-        const int l = lp[t];
-        if (l < prev) {
-            const double x = val[t];
-            int u = t;
-            for (; u > 0 && (int)lp[u - 1] > l; --u) {
-                lp[u] = lp[u - 1];
-                val[u] = val[u - 1];
-            }
-            lp[u] = (unsigned char)l;
-            val[u] = x;
-        } else {
-            prev = l;
-        }
-    }
-    prev = lp[0];
-    double cur = val[0];
-    unsigned pend = 0u;
-    int top = 0;
-    for (int t = 1; t < m; ++t) {
-        const int l = lp[t];
-        const double x = val[t];
-        const unsigned bit = 1u << (31 - __clz(prev ^ l));
-        unsigned low = pend & (bit - 1u);
-        pend = (pend & ~(bit - 1u)) | bit;
-        while (low) {
-            cur = fadd(val[--top], cur);
-            low &= low - 1u;
-        }
-        val[top++] = cur;
-        cur = x;
-        prev = l;
-    }
-    while (top > 0) cur = fadd(val[--top], cur);
-    return cur;
-}
 
 // The lane, as a value the compiler does not carry across rows: left alone it
 // keeps every lane-dependent address and bound of the row loop in a register
@@ -316,11 +261,6 @@ __device__ __forceinline__ void rm_products(const RmList& l, int ip, RmLists& ls
 template <int CAP>
 constexpr int rm_step() {
     return CAP <= 8 ? 1 : CAP / 8;
-}
-
-// Bits of w below bit b (b taken mod 32).
-__device__ __forceinline__ int popc_below(unsigned w, unsigned b) {
-    return __popc(__builtin_amdgcn_ubfe(w, 0u, b & 31u));
 }
 
 // Minimum and maximum of the products' columns over the wavefront.

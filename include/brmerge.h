@@ -157,7 +157,8 @@ int brm_flop_count_dev(const int *arpt, const int *acol, int64_t nnzA, const int
 /* Tuning knobs (names: "ws_budget_bytes", "med_cap", "leaf_cap",
  * "force_long", "profile", "lds_cfg", "group_cfg", "wmed_cap",
  * "wmed_engine", "launch_chunk", "cbar_budget_bytes", "sym_chunk_products",
- * "hash_cap", "upper_vm", "small_fused", "wmed_count", "wmed_bitmap");
+ * "hash_cap", "upper_vm", "small_fused", "wmed_count", "wmed_bitmap",
+ * "long_tiles");
  * returns BRM_E_INVALID for unknown names or
  * values.  Knobs other than hash_cap never change results, only speed.  group_cfg 0-3:
  * merge-path engine shapes for long rows; 4 (default): the bitmap-rank
@@ -181,7 +182,10 @@ int brm_flop_count_dev(const int *arpt, const int *acol, int64_t nnzA, const int
  * wavefront tier's row lengths are counted with column bitmaps; 0: with the
  * hash count.  wmed_bitmap (1, the default): the register tier ranks rows of
  * more than 128 products with column bitmaps (and takes rows of up to 2,048
- * products when B has at most 2^20 columns); 0: with a sort. */
+ * products when B has at most 2^20 columns); 0: with a sort.  long_tiles (1,
+ * the default): long rows of the bitmap-rank engine run in column tiles
+ * where the tables of B that takes pay; 0: never; 2 to 4,096: always, with
+ * that many column blocks. */
 int brm_set_param(const char *name, int64_t value);
 int64_t brm_get_param(const char *name);
 
