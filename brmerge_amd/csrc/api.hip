@@ -1166,11 +1166,7 @@ int run_small_g(const DevIn& in, int group, int64_t max_nnz, hipStream_t s, Phas
     }
     if (h.err) return dev_err_status(h.err, "small product");
     if (h.miss) return BRM_OK;
-    int64_t nnz = 0, ipt = 0;
-    for (int i = 0; i < SMALL_SLOTS; ++i) {
-        nnz += h.nnz[i];
-        ipt += h.ip[i];
-    }
+    const int64_t nnz = h.nnz, ipt = h.ip;
     sc.release(crpt);
     sc.release(ccol);
     sc.release(cval);

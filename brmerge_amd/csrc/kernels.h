@@ -93,14 +93,11 @@ int rmed_auto_cap(int N);
 
 // small.hip: products of at most SMALL_MAX_ROWS rows, all in the short tier.
 constexpr int SMALL_MAX_ROWS = 1 << 20;
-constexpr int SMALL_SLOTS = 32;  // partial-sum counters (summed by the host)
 struct SmallState {
     int err;     // DevErr bits
     int miss;    // a row has more than G lists or products: nothing of C is usable
-    int ticket;  // workgroup order of k_small
-    int pad;
-    int64_t nnz[SMALL_SLOTS];  // nnz(C), in partial sums
-    int64_t ip[SMALL_SLOTS];   // intermediate products, in partial sums
+    int64_t nnz;  // nnz(C)
+    int64_t ip;   // intermediate products
 };
 // int64 words of the state block (SmallState, then the look-back states)
 // for M rows in groups of `group` (32 or 64) lanes

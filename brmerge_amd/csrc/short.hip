@@ -41,36 +41,28 @@ __global__ __launch_bounds__(SH_NT) void k_short(const int* __restrict__ rows, i
         ip = (int)(a.ipA[a0 + L] - base);
     }
 
-    // list lanes (gl < L) load their list's product offset, B row start and
-    // A value; product gl finds its list p (largest p with off[p] <= gl) by
-    // a binary search over the group's lanes and takes p's descriptor by
-    // shuffles.  Rows with more lists than lanes search ipA in memory.
-    int off = INT_MAX, lbst = 0;
+    // list lanes (gl < L) load their list's product offsets, B row start and
+    // A value, and hand them to the list's products.  Rows with more lists
+    // than lanes search ipA in memory.
+    __shared__ ListSlot slots[SH_NT];
+    int off = 0, end = 0, lbst = 0;
     double lav = 0.0;
     if (gl < L) {
         off = (int)(a.ipA[a0 + gl] - base);
+        end = (int)(a.ipA[a0 + gl + 1] - base);
         lbst = a.brpt[a.acol[a0 + gl]];
         if (NUMERIC) lav = a.aval[a0 + gl];
     }
-    int p = 0;
-#pragma unroll
-    for (int step = G / 2; step >= 1; step >>= 1) {
-        const int cand = p + step;
-        const int oc = __shfl(off, gbase + (cand & (G - 1)), BRM_WAVE);
-        if (cand < L && oc <= gl) p = cand;
-    }
-    const int src = gbase + (p & (G - 1));
-    const int p_off = __shfl(off, src, BRM_WAVE);
-    const int p_bst = __shfl(lbst, src, BRM_WAVE);
-    const double p_av = __shfl(lav, src, BRM_WAVE);
+    const ListSlot ls = list_of<G>(&slots[threadIdx.x & ~(BRM_WAVE - 1)], gl, gbase, end > off, off, lbst, lav);
+    int p = ls.q;
     const bool act = gl < ip;
     int col = INT_MAX;
     double val = 0.0;
     if (act) {
         int bi;
-        double av = p_av;
+        double av = ls.av;
         if (L <= G) {
-            bi = p_bst + (gl - p_off);
+            bi = ls.rel + gl;
         } else {
             p = upper_idx(a.ipA + a0, 0, L, base + gl);
             const int ai = a0 + p;

@@ -7,22 +7,38 @@
 // ordered by position:
 //  - when the columns fit 32 - log2(G) bits, a bitonic sort of 32-bit keys
 //    (column, lane) over the group's lanes -- lanes are in list order, so
-//    within one column the lane order is the position order -- with DPP
-//    quad permutes for lane distances 1 and 2 and ds_swizzle for 4 to 16;
-//    each sorted lane then fetches its value and position from the lane its
-//    key names;
+//    within one column the lane order is the position order.  Every merge
+//    begins with the mirrored exchange (lane i with lane K-1-i), so that all
+//    exchanges ascend and one mask per lane bit selects the minimum or the
+//    maximum by v_med3; the exchanges are DPP moves up to distance 15 and
+//    ds_swizzle beyond.  Each sorted lane then fetches its value and position
+//    from the lane its key names;
 //  - otherwise a rank sort by 64-bit (column, position) keys (v_readlane
 //    broadcasts, or shuffles inside a half-wavefront), and ds_permute moves
 //    every lane's product to its rank.
 // The merge tree of BRMerge (BRMerge-SpGEMM/inc/spgemm.h:639-707: lists
 // paired (2j, 2j+1) level by level, odd list carried) is then evaluated
-// column-wise: at level l two live entries of the same column combine iff
-// their positions share the parent node (pos >> (l+1)); the left one keeps
-// the sum, the right one dies.  That is exactly the reference's value rule
-// -- an aligned binary tree over list positions in which a node with one
-// present child passes it through -- so the sums are bit-identical.
+// column-wise.  Entry j of a column joins the entries before it at the level
+// of the highest bit in which its position differs from that of entry j - 1
+// (the node that holds both), so each entry's level is known from one
+// neighbour; at level l the entries of that level add their value to the
+// nearest live entry on their left, which keeps the sum.  Which lanes receive
+// is found on the scalar unit, by the carries of one addition.  That is
+// exactly the reference's value rule -- an aligned binary tree over list
+// positions in which a node with one present child passes it through -- so
+// the sums are bit-identical.
+//
+// Bound by vector instructions: the sort takes two per exchange (three to
+// four as minimum, maximum and select) and a level a dozen (thirty when every
+// lane looks up its next live lane's column and position).  A * P of a
+// 27-point operator on 96^3 points with an aggregation, two rows of 27
+// products per wavefront and pass: 365 vector instructions per pass before,
+// 205 now.
 #pragma once
 #include "brm_device.h"
+#include "bucket_sum.h"
+
+#include <type_traits>
 
 namespace brm {
 
@@ -35,13 +51,23 @@ __device__ __forceinline__ double permute_f64(int dst_lane, double x) {
     return __hiloint2double(hi, lo);
 }
 
-// x of lane (this lane ^ J), within groups of 32 lanes (J < 64).
+// x of lane (this lane ^ J), for the distances the sort uses.
 template <int J>
 __device__ __forceinline__ uint32_t xor_lanes(uint32_t x) {
     if constexpr (J == 1) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
+        return (uint32_t)dpp_mov<0xB1, 0xF>((int)x, 0);  // quad_perm [1,0,3,2]
     } else if constexpr (J == 2) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
+        return (uint32_t)dpp_mov<0x4E, 0xF>((int)x, 0);  // quad_perm [2,3,0,1]
+    } else if constexpr (J == 3) {
+        return (uint32_t)dpp_mov<0x1B, 0xF>((int)x, 0);  // quad_perm [3,2,1,0]
+    } else if constexpr (J == 4) {
+        return xor_lanes<3>(xor_lanes<7>(x));
+    } else if constexpr (J == 7) {
+        return (uint32_t)dpp_mov<0x141, 0xF>((int)x, 0);  // row_half_mirror
+    } else if constexpr (J == 8) {
+        return (uint32_t)dpp_mov<0x128, 0xF>((int)x, 0);  // row_ror:8
+    } else if constexpr (J == 15) {
+        return (uint32_t)dpp_mov<0x140, 0xF>((int)x, 0);  // row_mirror
     } else if constexpr (J < 32) {
         return (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, 0x1F | (J << 10));  // bitmask mode, xor J
     } else {
@@ -49,20 +75,105 @@ __device__ __forceinline__ uint32_t xor_lanes(uint32_t x) {
     }
 }
 
-// One bitonic merge of blocks of K lanes (half-cleaners J = K/2 .. 1).
-template <int K, int J>
-__device__ __forceinline__ void bitonic_merge(uint32_t& key, int gl) {
+// One exchange at distance J: lanes with bit HALF of gl take the maximum.
+template <int J, int HALF>
+__device__ __forceinline__ uint32_t exchange(uint32_t key, int gl) {
     const uint32_t o = xor_lanes<J>(key);
-    const bool keep_min = ((gl & J) == 0) == ((gl & K) == 0);
-    key = keep_min ? min(key, o) : max(key, o);
-    if constexpr (J > 1) bitonic_merge<K, J / 2>(key, gl);
+    const uint32_t upper = (gl & HALF) ? 0xFFFFFFFFu : 0u;
+    return max(min(key, o), min(max(key, o), upper));  // v_med3_u32
+}
+
+template <int J>
+__device__ __forceinline__ void half_clean(uint32_t& key, int gl) {
+    key = exchange<J, J>(key, gl);
+    if constexpr (J > 1) half_clean<J / 2>(key, gl);
 }
 
 // Ascending sort of one key per lane over each group of G lanes.
 template <int K, int G>
 __device__ __forceinline__ void bitonic_sort(uint32_t& key, int gl) {
-    bitonic_merge<K, K / 2>(key, gl);
+    key = exchange<K - 1, K / 2>(key, gl);
+    if constexpr (K > 2) half_clean<K / 4>(key, gl);
     if constexpr (K < G) bitonic_sort<K * 2, G>(key, gl);
+}
+
+// Of two wavefront-uniform values the one of this lane's half (two vector
+// instructions, where a select of two scalars takes three).
+__device__ __forceinline__ uint32_t of_half(uint32_t lo, uint32_t hi, int gbase) {
+    const uint32_t m = (uint32_t)-(gbase >> 5);
+    return (lo & ~m) | (hi & m);
+}
+
+// The group's bits of a lane mask, and'ed with `with`: bit i is lane gbase + i.
+template <int G>
+__device__ __forceinline__ auto group_bits(uint64_t m, int gbase, std::conditional_t<G == BRM_WAVE, uint64_t, uint32_t> with) {
+    if constexpr (G == BRM_WAVE) {
+        return m & with;
+    } else {
+        const uint32_t h = (uint32_t)-(gbase >> 5);
+        return ((uint32_t)m & (with & ~h)) | ((uint32_t)(m >> 32) & (with & h));
+    }
+}
+
+// Lowest and highest set bit; any value when there is none.
+__device__ __forceinline__ int low_bit(uint32_t x) {
+    int r;
+    asm("v_ffbl_b32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+__device__ __forceinline__ int high_bit(uint32_t x) {
+    int r;
+    asm("v_ffbh_u32 %0, %1" : "=v"(r) : "v"(x));
+    return 31 - r;
+}
+
+// Number of set bits of m in the lanes below this one, of its group only.
+template <int G>
+__device__ __forceinline__ int group_rank(uint64_t m, int gbase) {
+    const int r = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    if constexpr (G == BRM_WAVE) return r;
+    else return r - (int)of_half(0u, __popc((unsigned)m), gbase);
+}
+
+// Inclusive sum over the lanes of each group.
+template <int G>
+__device__ __forceinline__ int group_incl_scan(int x) {
+    if constexpr (G == BRM_WAVE) return wave_incl_scan(x);
+    x += dpp_take<0x111, 0xF>(x);  // row_shr:1
+    x += dpp_take<0x112, 0xF>(x);  // row_shr:2
+    x += dpp_take<0x114, 0xF>(x);  // row_shr:4
+    x += dpp_take<0x118, 0xF>(x);  // row_shr:8
+    return x + dpp_take<0x142, 0xA>(x);  // row_bcast15 into rows 1 and 3
+}
+
+// The list of each product lane: lists of one row (list q of the group in
+// its lane q) are laid out one after the other over the group's lanes.
+struct alignas(16) ListSlot {
+    int q;       // list
+    int rel;     // index in B of the product less its lane
+    double av;   // A value
+};
+// ne: this lane's list is not empty and begins at product off < G.  ws: the
+// wavefront's 64 slots in LDS.  Product lanes (below the row's products) get
+// their list's slot; other lanes any slot.
+template <int G>
+__device__ __forceinline__ ListSlot list_of(ListSlot* ws, int gl, int gbase, bool ne, int off, int bst, double av) {
+    ws[gbase + gl].q = -1;
+    wave_lds_sync();
+    if (ne) ws[gbase + off] = ListSlot{gl, bst - off, av};
+    wave_lds_sync();
+    const uint64_t begins = __ballot(ws[gbase + gl].q >= 0);
+    // last list begin at or before this lane
+    int s;
+    if constexpr (G == BRM_WAVE) {
+        const uint64_t b = begins & (~0ull >> (BRM_WAVE - 1 - gl));
+        s = b ? 63 - __clzll((long long)b) : 0;
+    } else {
+        s = high_bit(group_bits<G>(begins, gbase, ~0u >> (31 - gl)));
+    }
+    const ListSlot r = ws[gbase + (s & (G - 1))];
+    wave_lds_sync();
+    return r;
 }
 
 // Whether columns below N fit the 32-bit sort keys of groups of G lanes
@@ -93,7 +204,7 @@ __device__ __forceinline__ ShortMerged short_merge(int col, int p, double val, b
                                                    uint64_t gmask, bool narrow) {
     const int lane = lane_id();
     constexpr int S = G == 64 ? 6 : 5;
-    bool alive = gl < ip;
+    const bool alive = gl < ip;
     int pos;
     if (narrow) {
         uint32_t key = act ? (((uint32_t)col << S) | (uint32_t)gl) : 0xFFFFFFFFu;
@@ -147,32 +258,40 @@ __device__ __forceinline__ ShortMerged short_merge(int col, int p, double val, b
         val = permute_f64(dst, val);
     }
 
-    const uint64_t below_me = (1ull << lane) - 1ull;
-    const uint64_t above_me = lane == BRM_WAVE - 1 ? 0ull : ~0ull << (lane + 1);
-    for (int l = 0; l < 31; ++l) {
-        const uint64_t am = __ballot(alive) & gmask;
-        const uint64_t above = am & above_me;
-        const int nxt = above ? (__ffsll((long long)above) - 1) : lane;
-        const int ncol = __shfl(col, nxt, BRM_WAVE);
-        const int npos = __shfl(pos, nxt, BRM_WAVE);
-        const double nval = __shfl(val, nxt, BRM_WAVE);
-        const bool same = alive && above != 0ull && ncol == col;
-        if (__ballot(same) == 0ull) break;  // no column left to combine in any group
-        const bool comb = same && ((npos >> (l + 1)) == (pos >> (l + 1)));
-        const uint64_t cm = __ballot(comb);
-        const uint64_t below = am & below_me;
-        const int prv = below ? (63 - __clzll((long long)below)) : -1;
-        const bool dies = prv >= 0 && ((cm >> prv) & 1ull);
-        if (comb) val = fadd(val, nval);
-        alive = alive && !dies;
+    // ---- the tree: lvl is the level at which this entry joins the one on its left
+    const int pcol = dpp_mov<0x138, 0xF>(col, 0);  // wave_shr:1
+    const int ppos = dpp_mov<0x138, 0xF>(pos, 0);
+    const bool joins = alive && gl > 0 && pcol == col;
+    int lvl = joins ? 31 - __clz(pos ^ ppos) : -1;  // positions of one column differ
+    asm volatile("" : "+v"(lvl));  // compared as it is, not by its parts
+    uint64_t am = __ballot(alive), todo = __ballot(joins);
+    for (int l = 0; todo != 0ull; ++l) {
+        const uint64_t die = __ballot(lvl == l);
+        if (die == 0ull) continue;
+        todo &= ~die;
+        // the live lane before each of `die`: in reversed order a carry from
+        // each runs through the dead lanes and stops at the next live one
+        // (two entries of one level never follow each other)
+        const uint64_t rl = __brevll(am);
+        const bool gets = __builtin_amdgcn_inverse_ballot_w64(__brevll((~rl + (__brevll(die) << 1)) & rl));
+        int nxt;  // byte address of the next lane of `die` (a lane that gets is not in it)
+        if constexpr (G == BRM_WAVE) {
+            nxt = (__ffsll((long long)(die & (~0ull << gl))) - 1) << 2;
+        } else {
+            nxt = (low_bit(group_bits<G>(die, gbase, ~0u << gl)) << 2) + (gbase << 2);
+        }
+        const int nlo = __builtin_amdgcn_ds_bpermute(nxt, __double2loint(val));  // address modulo 256
+        const int nhi = __builtin_amdgcn_ds_bpermute(nxt, __double2hiint(val));
+        if (gets) val = fadd(val, __hiloint2double(nhi, nlo));
+        am &= ~die;
     }
-    const uint64_t am = __ballot(alive) & gmask;
     ShortMerged r{};
     r.col = col;
     r.val = val;
-    r.alive = alive;
-    r.idx = __popcll(am & below_me);
-    r.nout = __popcll(am);
+    r.alive = __builtin_amdgcn_inverse_ballot_w64(am);
+    r.idx = group_rank<G>(am, gbase);
+    if constexpr (G == BRM_WAVE) r.nout = __popcll(am);
+    else r.nout = (int)of_half(__popc((uint32_t)am), __popc((uint32_t)(am >> 32)), gbase);
     return r;
 }
 

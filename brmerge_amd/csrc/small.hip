@@ -3,22 +3,20 @@
 // A product whose rows are all short (at most G = 64, or 32, lists and
 // products) spends more on the general pipeline's dozen launches and two
 // host round trips than on its kernels.  Such a product runs as:
-//   1. one fill clearing the state: flags, counters, workgroup tickets and
-//      look-back states;
-//   2. k_small<G>: each workgroup takes a ticket (tickets are handed out in
-//      the order workgroups start) and with it a run of consecutive rows,
-//      in P passes of one row per group of G lanes.  The passes are
-//      batched stage by stage -- all row pointers, then all list
-//      descriptors, then all B entries -- so that each dependent load is
-//      issued for every pass before the first one is waited on.  Each group
-//      checks its rows' own indices, finds the list offsets by a group scan
-//      (no global product scan) and merges the row in registers with the
-//      short tier's code (short_merge.h).  The workgroup's nnz is scanned
-//      across workgroups by decoupled look-back (a workgroup waits only on
-//      workgroups that started before it), and every row is written straight
-//      from registers into C at its place, with C's row pointer.
-//      Workgroups past the row workgroups check all of B, one B row per
-//      thread (row pointers, column range, sorted rows), as the general
+//   1. one fill clearing the state: flags, totals and the words through
+//      which the workgroups' places in C are handed on;
+//   2. k_small<G, P>: each workgroup takes a run of consecutive rows, in P
+//      passes of one row per group of G lanes.  The passes are batched stage
+//      by stage -- all row pointers, then all list descriptors, then all B
+//      entries -- so that each dependent load is issued for every pass before
+//      the first one is waited on.  Each group checks its rows' own indices,
+//      finds the list offsets by a group scan (no global product scan) and
+//      merges the row in registers with the short tier's code
+//      (short_merge.h).  Every workgroup publishes its nnz, one wavefront of
+//      the grid scans these as they come and publishes each workgroup's place,
+//      and every row is written straight from registers into C, with C's row
+//      pointer.  Workgroups past the row workgroups check all of B, one B row
+//      per thread (row pointers, column range, sorted rows), as the general
 //      validation does.
 // C is allocated beforehand for G entries per row, a bound of nnz(C) when
 // every row is short.  The host reads the state once, at the end: a row with
@@ -35,77 +33,115 @@
 namespace brm {
 namespace {
 
-// Look-back states: bits 62-63 the state (1: aggregate, 2: inclusive
-// prefix), bits 0-61 the value.  Each state word carries its own value, so
-// relaxed atomics (no cache invalidation or write-back) are enough.
-constexpr uint64_t LB_AGG = 1ull << 62, LB_INC = 2ull << 62, LB_VAL = (1ull << 62) - 1ull;
+// Two words per row workgroup, cleared beforehand: what it adds (own) and
+// what comes before it (pre).  The top bit marks a word as published; below
+// it products (from bit SC_IP) and nnz(C), both under 2^31.  Each word
+// carries its own value, so relaxed atomics (no cache invalidation or
+// write-back) are enough.
+constexpr int SC_IP = 31;
+constexpr uint64_t SC_SET = 1ull << 63, SC_LATE = 1ull << 62, SC_VAL = SC_LATE - 1ull;
+static_assert((int64_t)SMALL_MAX_ROWS * BRM_WAVE < ((int64_t)1 << SC_IP), "two counts in a word");
+constexpr int SC_POLLS = 1 << 14;
 
-// Exclusive prefix of this workgroup's `agg` over the workgroups before
-// ticket b; called by all of wavefront 0.  Lane l reads the state l + 1
-// below the window's top, 64 states per step.
-__device__ int64_t look_back(uint64_t* lb, int b, int64_t agg) {
+__device__ __forceinline__ uint64_t sc_load(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void sc_store(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The scanner (one wavefront, workgroup 0): reads the workgroups' own words
+// in order as they appear and publishes each one's prefix.  A row workgroup
+// then waits for one word.  (Decoupled look-back, every workgroup reading back
+// to the nearest prefix, had the thousand resident workgroups poll the same
+// cache lines past the L2 caches: with it A * P of a 27-point operator on 96^3
+// points and an aggregation took 272 us, with the scanner 210, without any
+// wait 180.)
+// Workgroups start about in the order of their index, but nothing promises
+// it, so both waits are bounded: after SC_POLLS looks without a new word the
+// scanner marks the rest late, and the product is left to the general
+// pipeline.
+__device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nb) {
     const int lane = lane_id();
-    int64_t prefix = 0;
-    if (b > 0) {
-        if (lane == 0) __hip_atomic_store(&lb[b], LB_AGG | (uint64_t)agg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int hi = b - 1;;) {
-            const int q = hi - lane;
-            const uint64_t v = q >= 0 ? __hip_atomic_load(&lb[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                      : LB_INC;  // before workgroup 0: an empty prefix
-            const uint64_t incm = __ballot((v & ~LB_VAL) == LB_INC);
-            const int first = incm ? __ffsll((long long)incm) - 1 : BRM_WAVE;  // nearest prefix
-            const uint64_t upto = first >= BRM_WAVE - 1 ? ~0ull : ((2ull << first) - 1ull);
-            if ((__ballot(v == 0) & upto) != 0ull) {  // a state not yet published
-                __builtin_amdgcn_s_sleep(1);
-                continue;
-            }
-            prefix += wave_sum((lane <= first) ? (int64_t)(v & LB_VAL) : (int64_t)0);
-            if (first < BRM_WAVE) break;
-            hi -= BRM_WAVE;
+    uint64_t sum = 0;
+    int polls = 0;
+    for (int base = 0; base < nb;) {
+        const uint64_t v = sc_load(&own[min(base + lane, nb - 1)]);
+        const uint64_t gap = __ballot((v & SC_SET) == 0 || base + lane >= nb);
+        const int got = gap ? __ffsll((long long)gap) - 1 : BRM_WAVE;  // words up to the first unpublished one
+        if (got == 0) {
+            if (++polls <= SC_POLLS) continue;
+            for (int q = base + lane; q < nb; q += BRM_WAVE) sc_store(&pre[q], SC_SET | SC_LATE);
+            return;
         }
+        polls = 0;
+        const uint64_t mine = lane < got ? v & SC_VAL : 0;
+        const uint64_t inc = wave_incl_scan(mine);
+        if (lane < got) sc_store(&pre[base + lane], SC_SET | (sum + inc - mine));
+        sum += wave_last(inc);
+        base += got;
     }
-    if (lane == 0)
-        __hip_atomic_store(&lb[b], LB_INC | (uint64_t)(prefix + agg), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return prefix;
+}
+
+// The prefix of workgroup b (called by one wavefront); 0 and *late when it
+// does not come.
+__device__ uint64_t await_prefix(uint64_t* own, const uint64_t* pre, int b, uint64_t mine, bool* late) {
+    if (lane_id() == 0) sc_store(&own[b], SC_SET | mine);
+    for (int polls = 0; polls < 4 * SC_POLLS; ++polls) {
+        const uint64_t v = sc_load(&pre[b]);
+        if (v & SC_SET) {
+            *late = (v & SC_LATE) != 0;
+            return *late ? 0 : v & SC_VAL;
+        }
+        __builtin_amdgcn_s_sleep(2);
+    }
+    *late = true;
+    return 0;
 }
 
 // Workgroup shape per group size: threads and passes.  A workgroup takes
 // RPP * P consecutive rows (RPP rows per pass); wavefront 0 scans them, R per
-// lane.  More rows per workgroup means fewer look-back states to chain.
-constexpr int SM_NT32 = 512, SM_P32 = 4;   // G = 32
-constexpr int SM_NT64 = 1024, SM_P64 = 4;  // G = 64
+// lane.
+constexpr int SM_NT32 = 512;   // G = 32
+constexpr int SM_NT64 = 1024;  // G = 64
+constexpr int SM_P = 4;
 // B rows longer than this are left to the general pipeline's validation.
 constexpr int SM_BROW_MAX = 64;
 
-template <int G>
+template <int G, int P_>
 struct SmallShape {
     static constexpr int NT = G == 32 ? SM_NT32 : SM_NT64;  // threads
-    static constexpr int P = G == 32 ? SM_P32 : SM_P64;     // passes
+    static constexpr int P = P_;                             // passes
     static constexpr int WPB = NT / BRM_WAVE;                // wavefronts
     static constexpr int RPW = BRM_WAVE / G;                 // rows per wavefront and pass
     static constexpr int RPP = WPB * RPW;                    // rows per pass
     static constexpr int ROWS = RPP * P;                     // rows per workgroup
-    static constexpr int R = ROWS / BRM_WAVE;                // rows per lane of the scan
-    static_assert(R * BRM_WAVE == ROWS && R >= 1, "row layout");
+    static constexpr int R = (ROWS + BRM_WAVE - 1) / BRM_WAVE;  // rows per lane of the scan
+    static_assert(R * BRM_WAVE == ROWS || ROWS < BRM_WAVE, "row layout");
 };
 
-template <int G>
-__global__ __launch_bounds__(SmallShape<G>::NT) void k_small(RowArgs a, int64_t nnzA, int64_t nnzB, int row_blocks,
+template <int G, int P>
+__global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int nnzA, int nnzB, int row_blocks,
                                                               int64_t* __restrict__ crpt, int* __restrict__ ccol,
                                                               double* __restrict__ cval, SmallState* __restrict__ st,
-                                                              uint64_t* __restrict__ lb) {
-    using S = SmallShape<G>;
-    constexpr int P = S::P;
+                                                              uint64_t* __restrict__ own) {
+    using S = SmallShape<G, P>;
     const int lane = lane_id();
     const int w = (int)(threadIdx.x / BRM_WAVE);
-    if ((int)blockIdx.x >= row_blocks) {
+    uint64_t* pre = own + row_blocks;
+    if (blockIdx.x == 0) {
+        if (w == 0) scan_workgroups(own, pre, row_blocks);
+        return;
+    }
+    const int b = (int)blockIdx.x - 1;
+    if (b >= row_blocks) {
         // ---- B: one row per thread; entries 8 at a time (indices clamped
         // into the row, so that every load is in bounds)
-        const int r = ((int)blockIdx.x - row_blocks) * S::NT + (int)threadIdx.x;
+        const int r = (b - row_blocks) * S::NT + (int)threadIdx.x;
         bool bad = false, lng = false;
         if (r < a.K) {
             const int b0 = a.brpt[r], b1 = a.brpt[r + 1];
-            if (b0 < 0 || b0 > b1 || (int64_t)b1 > nnzB) {
+            if (b0 < 0 || b0 > b1 || b1 > nnzB) {
                 bad = true;
             } else if (b1 - b0 > SM_BROW_MAX) {
                 lng = true;
@@ -125,24 +161,21 @@ __global__ __launch_bounds__(SmallShape<G>::NT) void k_small(RowArgs a, int64_t 
                 }
             }
         } else if (r == a.K) {
-            bad = a.brpt[0] != 0 || (int64_t)a.brpt[a.K] != nnzB;
+            bad = a.brpt[0] != 0 || a.brpt[a.K] != nnzB || a.arpt[0] != 0 || a.arpt[a.M] != nnzA;
         }
         if (__ballot(bad) != 0ull && lane == 0) atomicOr(&st->err, (int)DERR_INVALID);
         if (__ballot(lng) != 0ull && lane == 0) atomicOr(&st->miss, 1);
         return;
     }
-    __shared__ int ticket;
     __shared__ int rcnt[S::ROWS];      // nnz of the workgroup's rows
     __shared__ int rip[S::ROWS];       // their products
     __shared__ int64_t rbase[S::ROWS];  // their C offsets
-    if (threadIdx.x == 0) ticket = atomicAdd(&st->ticket, 1);
-    __syncthreads();
-    const int b = ticket;
+    __shared__ ListSlot slots[S::NT];
     const int gl = lane & (G - 1);
     const int gbase = lane & ~(G - 1);
-    const uint64_t gmask = G == BRM_WAVE ? ~0ull : (((1ull << G) - 1ull) << gbase);
+    const uint64_t gmask = (~0ull >> (BRM_WAVE - G)) << gbase;
     const int slot = w * S::RPW + lane / G;  // the group's row within a pass
-    bool bad = false, miss = false;          // group-uniform
+    bool bad = false, miss = false;
     // ---- stage 1: row pointers (all passes' loads first), checked before
     // they are followed; the checks use | and & so that no branch separates
     // one pass's loads from the next
@@ -158,8 +191,7 @@ __global__ __launch_bounds__(SmallShape<G>::NT) void k_small(RowArgs a, int64_t 
     for (int p = 0; p < P; ++p) {
         const int row = b * S::ROWS + p * S::RPP + slot;
         const bool has = row < a.M;
-        const bool rb = has & ((a0[p] < 0) | (a0[p] > a1[p]) | ((int64_t)a1[p] > nnzA) | ((row == 0) & (a0[p] != 0)) |
-                               ((row == a.M - 1) & ((int64_t)a1[p] != nnzA)));
+        const bool rb = has & ((a0[p] < 0) | (a0[p] > a1[p]) | (a1[p] > nnzA));
         const bool ms = has & !rb & (a1[p] - a0[p] > G);
         bad |= rb;
         miss |= ms;
@@ -183,41 +215,28 @@ __global__ __launch_bounds__(SmallShape<G>::NT) void k_small(RowArgs a, int64_t 
         lbst[p] = a.brpt[cc];
         lend[p] = a.brpt[cc + 1];
     }
-    // ---- stage 3: list offsets, each lane's product, its B entry
+    // ---- stage 3: list offsets, each lane's product, its B entry.  A list
+    // that is malformed or longer than G counts as G + 1 entries: its row is
+    // not merged, and the group's sum stays within int
     int pl[P], bcl[P], ipn[P];
     double pav[P], bvl[P];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const bool v = gl < L[p];
         const bool lbad = v & ((acl[p] < 0) | (acl[p] >= a.K) | (lbst[p] < 0) | (lbst[p] > lend[p]) |
-                               ((int64_t)lend[p] > nnzB));
-        const bool gbad = (__ballot(lbad) & gmask) != 0ull;
-        bad |= gbad;
-        // lengths capped at G + 1: a longer row is a miss either way, and the
-        // group's sum stays within int
-        const int bl = (v & !gbad) ? min(lend[p] - lbst[p], G + 1) : 0;
-        int incl = wave_incl_scan(bl);
-        if (G < BRM_WAVE) incl -= __shfl(incl, (gbase + BRM_WAVE - 1) & (BRM_WAVE - 1), BRM_WAVE) * (gbase > 0);
-        const int ip = __shfl(incl, gbase + G - 1, BRM_WAVE);
-        const bool ms = ok[p] & !gbad & (ip > G);
-        miss |= ms;
-        const bool run = ok[p] & !gbad & !ms;
-        ipn[p] = run ? ip : 0;
-        const int off = v ? incl - bl : INT_MAX;
-        // product lane -> its list (largest q with off[q] <= gl), as the short tier
-        int q = 0;
-#pragma unroll
-        for (int step = G / 2; step >= 1; step >>= 1) {
-            const int cand = q + step;
-            const int oc = __shfl(off, gbase + (cand & (G - 1)), BRM_WAVE);
-            if (cand < L[p] && oc <= gl) q = cand;
-        }
-        const int src = gbase + (q & (G - 1));
-        const int q_off = __shfl(off, src, BRM_WAVE);
-        const int q_bst = __shfl(lbst[p], src, BRM_WAVE);
-        pav[p] = __shfl(lav[p], src, BRM_WAVE);
-        pl[p] = q;
-        const int bi = gl < ipn[p] ? q_bst + (gl - q_off) : 0;  // nnz(B) >= 1
+                               (lend[p] > nnzB));
+        bad |= lbad;
+        const int bl = v ? (lbad ? G + 1 : min(lend[p] - lbst[p], G + 1)) : 0;
+        const int incl = group_incl_scan<G>(bl);
+        int ip = __builtin_amdgcn_readlane(incl, BRM_WAVE - 1);
+        if (G < BRM_WAVE) ip = (int)of_half((uint32_t)__builtin_amdgcn_readlane(incl, G - 1), (uint32_t)ip, gbase);
+        miss |= ip > G;
+        ipn[p] = ip > G ? 0 : ip;
+        const int off = incl - bl;
+        const ListSlot ls = list_of<G>(&slots[w * BRM_WAVE], gl, gbase, (bl > 0) & (off < G), off, lbst[p], lav[p]);
+        pl[p] = ls.q;
+        pav[p] = ls.av;
+        const int bi = gl < ipn[p] ? ls.rel + gl : 0;  // nnz(B) >= 1
         bcl[p] = a.bcol[bi];
         bvl[p] = a.bval[bi];
     }
@@ -237,33 +256,38 @@ __global__ __launch_bounds__(SmallShape<G>::NT) void k_small(RowArgs a, int64_t 
     if (__ballot(bad) != 0ull && lane == 0) atomicOr(&st->err, (int)DERR_INVALID);
     if (__ballot(miss) != 0ull && lane == 0) atomicOr(&st->miss, 1);
     __syncthreads();
-    // ---- the workgroup's rows in C: a scan over its rows, look-back over
-    // the workgroups before it; C's row pointer from wavefront 0
+    // ---- the workgroup's rows in C: a scan over its rows, behind the
+    // workgroups before it; C's row pointer from wavefront 0
     if (w == 0) {
         int64_t local = 0, ips = 0;
 #pragma unroll
         for (int j = 0; j < S::R; ++j) {
+            if (lane * S::R + j >= S::ROWS) continue;
             local += rcnt[lane * S::R + j];
             ips += rip[lane * S::R + j];
         }
         const int64_t inc = wave_incl_scan(local);
         const int64_t agg = wave_last(inc);
         ips = wave_sum(ips);
-        const int64_t base = look_back(lb, b, agg);
+        bool late = false;
+        const uint64_t before = await_prefix(own, pre, b, ((uint64_t)ips << SC_IP) | (uint64_t)agg, &late);
+        const int64_t base = (int64_t)(before & ((1ull << SC_IP) - 1ull));
         int64_t off = base + inc - local;
 #pragma unroll
         for (int j = 0; j < S::R; ++j) {
             const int k = lane * S::R + j;
+            if (k >= S::ROWS) continue;
             const int row = b * S::ROWS + k;
             rbase[k] = off;
             if (row < a.M) crpt[row] = off;
             off += rcnt[k];
             if (row == a.M - 1) crpt[a.M] = off;
         }
-        // nnz(C) and the products: one atomic each per workgroup, spread over
-        // SMALL_SLOTS counters so that no address is hot
-        if (lane == 0 && agg) atomicAdd((unsigned long long*)&st->nnz[b % SMALL_SLOTS], (unsigned long long)agg);
-        if (lane == 1 && ips) atomicAdd((unsigned long long*)&st->ip[b % SMALL_SLOTS], (unsigned long long)ips);
+        if (lane == 0 && late) atomicOr(&st->miss, 1);
+        if (lane == 0 && b == row_blocks - 1) {
+            st->nnz = base + agg;
+            st->ip = (int64_t)(before >> SC_IP) + ips;
+        }
     }
     __syncthreads();
 #pragma unroll
@@ -276,28 +300,56 @@ __global__ __launch_bounds__(SmallShape<G>::NT) void k_small(RowArgs a, int64_t 
     }
 }
 
-template <int G>
+template <int G, int P>
 int64_t row_blocks_of(int M) {
-    return ((int64_t)M + SmallShape<G>::ROWS - 1) / SmallShape<G>::ROWS;
+    return ((int64_t)M + SmallShape<G, P>::ROWS - 1) / SmallShape<G, P>::ROWS;
+}
+
+template <int G, int P>
+hipError_t launch_small_gp(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
+                           SmallState* st, uint64_t* own, hipStream_t s) {
+    using S = SmallShape<G, P>;
+    const int64_t rb = row_blocks_of<G, P>(a.M);
+    const int64_t bb = ((int64_t)a.K + 1 + S::NT - 1) / S::NT;
+    if (1 + rb + bb > INT32_MAX || nnzA > INT32_MAX || nnzB > INT32_MAX) return hipErrorInvalidValue;
+    ProfScope ps_("k_small", s);
+    k_small<G, P><<<(unsigned)(1 + rb + bb), S::NT, 0, s>>>(a, (int)nnzA, (int)nnzB, (int)rb, crpt, ccol, cval, st, own);
+    return hipGetLastError();
+}
+
+// Passes per workgroup: the fewest that leave at most SM_FEW workgroups (two
+// per CU), else SM_P.  Few rows are a matter of latency, which passes add to;
+// many workgroups a matter of handing the places on, 8 ns each.  k_small, us:
+//   rows     products each | P = 1    2      4      8
+//   2,048    64            | 7.3             10.6
+//   16,384   64            | 19.9     15.5   17.6
+//   884,736  27            |          327    210    247
+constexpr int SM_FEW = 512;
+template <int G>
+int passes_of(int M) {
+    return row_blocks_of<G, 1>(M) <= SM_FEW ? 1 : row_blocks_of<G, 2>(M) <= SM_FEW ? 2 : SM_P;
 }
 
 template <int G>
 hipError_t launch_small_g(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
-                          SmallState* st, uint64_t* lb, hipStream_t s) {
-    using S = SmallShape<G>;
-    const int64_t rb = row_blocks_of<G>(a.M);
-    const int64_t bb = ((int64_t)a.K + 1 + S::NT - 1) / S::NT;
-    if (rb + bb > INT32_MAX) return hipErrorInvalidValue;
-    ProfScope ps_("k_small", s);
-    k_small<G><<<(unsigned)(rb + bb), S::NT, 0, s>>>(a, nnzA, nnzB, (int)rb, crpt, ccol, cval, st, lb);
-    return hipGetLastError();
+                          SmallState* st, uint64_t* own, hipStream_t s) {
+    switch (passes_of<G>(a.M)) {
+        case 1: return launch_small_gp<G, 1>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
+        case 2: return launch_small_gp<G, 2>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
+        default: return launch_small_gp<G, SM_P>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
+    }
+}
+
+template <int G>
+int64_t states_of(int M) {
+    const int p = passes_of<G>(M);
+    return p == 1 ? row_blocks_of<G, 1>(M) : p == 2 ? row_blocks_of<G, 2>(M) : row_blocks_of<G, SM_P>(M);
 }
 
 }  // namespace
 
 int64_t small_state_words(int M, int group) {
-    const int64_t nb = group == 32 ? row_blocks_of<32>(M) : row_blocks_of<64>(M);
-    return (int64_t)(sizeof(SmallState) / 8) + nb;
+    return (int64_t)(sizeof(SmallState) / 8) + 2 * (group == 32 ? states_of<32>(M) : states_of<64>(M));
 }
 
 hipError_t launch_small(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
@@ -305,9 +357,9 @@ hipError_t launch_small(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* c
     if (a.M < 1 || a.K < 1 || nnzA < 1 || nnzB < 1) return hipErrorInvalidValue;
     hipError_t e = launch_fill_i64((int64_t*)st, small_state_words(a.M, group), 0, s);
     if (e != hipSuccess) return e;
-    uint64_t* lb = reinterpret_cast<uint64_t*>(st) + sizeof(SmallState) / 8;
-    return group == 32 ? launch_small_g<32>(a, nnzA, nnzB, crpt, ccol, cval, st, lb, s)
-                       : launch_small_g<64>(a, nnzA, nnzB, crpt, ccol, cval, st, lb, s);
+    uint64_t* own = reinterpret_cast<uint64_t*>(st) + sizeof(SmallState) / 8;
+    return group == 32 ? launch_small_g<32>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s)
+                       : launch_small_g<64>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
 }
 
 }  // namespace brm
