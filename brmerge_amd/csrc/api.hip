@@ -143,19 +143,25 @@ void PhaseClock::collect(double* out) {
 // Small read-backs go through a pinned buffer of the calling thread (a copy
 // into pageable memory is staged by the runtime and takes longer), several
 // of them behind one synchronisation.  The buffer is kept until the process
-// ends.
+// ends.  k_small writes its result there itself (a thread has one call under
+// way at a time).
 constexpr size_t D2H_PINNED = 4096;
 
-int d2h_parts(std::initializer_list<D2HPart> parts, hipStream_t s) {
+static unsigned char* thread_pinned() {  // nullptr when there is none to be had
     static thread_local unsigned char* pinned = nullptr;
-    size_t tot = 0;
-    for (const D2HPart& q : parts) tot += (q.bytes + 15) & ~(size_t)15;
-    if (tot <= D2H_PINNED && !pinned) {
+    if (!pinned) {
         void* ptr = nullptr;
         if (hipHostMalloc(&ptr, D2H_PINNED, hipHostMallocDefault) == hipSuccess) pinned = (unsigned char*)ptr;
         else (void)hipGetLastError();
     }
-    if (tot > D2H_PINNED || !pinned) {
+    return pinned;
+}
+
+int d2h_parts(std::initializer_list<D2HPart> parts, hipStream_t s) {
+    size_t tot = 0;
+    for (const D2HPart& q : parts) tot += (q.bytes + 15) & ~(size_t)15;
+    unsigned char* const pinned = tot <= D2H_PINNED ? thread_pinned() : nullptr;
+    if (!pinned) {
         for (const D2HPart& q : parts) HIPC(hipMemcpyAsync(q.dst, q.src, q.bytes, hipMemcpyDeviceToHost, s));
         HIPC(hipStreamSynchronize(s));
         return BRM_OK;
@@ -1137,12 +1143,14 @@ int run_small_g(const DevIn& in, int group, int64_t max_nnz, hipStream_t s, Phas
     const int64_t cap = (int64_t)M * group;
     if (cap > max_nnz) return BRM_OK;
     Scratch sc;
-    SmallState* st;
+    SmallResult* const res = reinterpret_cast<SmallResult*>(thread_pinned());
+    if (!res) return BRM_OK;
+    int64_t* words;
     int64_t* crpt;
     int* ccol;
     double* cval;
     clk.begin(P_PRE);
-    BRMC(sc.alloc(reinterpret_cast<int64_t**>(&st), small_state_words(M, group), "small-product state"));
+    BRMC(sc.alloc(&words, small_words(M, in.K, group), "small-product words"));
     BRMC(sc.alloc(&crpt, (int64_t)M + 1, "crpt"));
     BRMC(sc.alloc(&ccol, cap, "C col"));
     BRMC(sc.alloc(&cval, cap, "C val"));
@@ -1157,15 +1165,12 @@ int run_small_g(const DevIn& in, int group, int64_t max_nnz, hipStream_t s, Phas
     a.K = in.K;
     a.N = in.N;
     clk.begin(P_COMPUTE);
-    HIPC(launch_small(a, in.nnzA, in.nnzB, crpt, ccol, cval, st, group, s));
-    SmallState h{};
-    BRMC(d2h(&h, st, sizeof(h), s));
-    if (h.err & DERR_INVALID) {
-        set_err("validation: malformed CSR input (row pointers, column range or unsorted/duplicate B columns)");
-        return BRM_E_INVALID;
-    }
-    if (h.err) return dev_err_status(h.err, "small product");
-    if (h.miss) return BRM_OK;
+    *res = SmallResult{};
+    HIPC(launch_small(a, in.nnzA, in.nnzB, crpt, ccol, cval, res, reinterpret_cast<uint64_t*>(words), group, s));
+    HIPC(hipStreamSynchronize(s));
+    const SmallResult h = *res;
+    if (h.bad) return dev_err_status(DERR_INVALID, "validation");
+    if (!h.done || h.miss || h.late) return BRM_OK;
     const int64_t nnz = h.nnz, ipt = h.ip;
     sc.release(crpt);
     sc.release(ccol);
@@ -1199,6 +1204,8 @@ int run_small(const DevIn& in, double avg_ip, int64_t max_nnz, hipStream_t s, Ph
 
 int run_spgemm(const DevIn& in, bool upper, int64_t max_nnz, hipStream_t s, DevOut* out, double* ph,
                const ExtOut* ext) {
+    // A caller that asks for no phase times pays for none: the clock's events
+    // take 31 us of a product of 2,048 short rows that takes 24 without.
     PhaseClock clk(s, ph != nullptr);
     memset(&t_stats, 0, sizeof(t_stats));
     HostTrace tr(s);
@@ -1218,11 +1225,13 @@ int run_spgemm(const DevIn& in, bool upper, int64_t max_nnz, hipStream_t s, DevO
         params().hash_cap == 0 && avg_l * avg_b <= 64.0) {
         bool handled = false;
         BRMC(run_small(in, avg_l * avg_b, max_nnz, s, clk, out, &handled));
-        if (handled) {
-            clk.begin(P_CLEAN);
-            HIPC(hipStreamSynchronize(s));
-            clk.end();
-            if (ph) clk.collect(ph);
+        if (handled) {  // the stream has been waited for
+            if (ph) {
+                clk.begin(P_CLEAN);
+                clk.end();
+                HIPC(hipStreamSynchronize(s));
+                clk.collect(ph);
+            }
             dev_flush_deferred();
             return BRM_OK;
         }
@@ -1296,8 +1305,10 @@ int run_spgemm(const DevIn& in, bool upper, int64_t max_nnz, hipStream_t s, DevO
     clk.begin(P_CLEAN);
     HIPC(hipStreamSynchronize(s));
     clk.end();
-    HIPC(hipStreamSynchronize(s));
-    if (ph) clk.collect(ph);
+    if (ph) {
+        HIPC(hipStreamSynchronize(s));
+        clk.collect(ph);
+    }
 
     t_stats.nnz_c = nnzC;
     sc.release(p.crpt);
@@ -1463,7 +1474,7 @@ int dev_entry(const int* arpt, const int* acol, const double* aval, int64_t nnzA
     DevIn in{arpt, acol, aval, nnzA, brpt, bcol, bval, nnzB, M, K, N};
     DevOut out{};
     double ph[P_N] = {0};
-    BRMC(run_spgemm(in, upper, INT64_MAX, (hipStream_t)stream, &out, ph));
+    BRMC(run_spgemm(in, upper, INT64_MAX, (hipStream_t)stream, &out, timing ? ph : nullptr));
     *crpt = out.crpt;
     *ccol = out.ccol;
     *cval = out.cval;
@@ -1501,7 +1512,8 @@ int brm_spgemm_precise_i32(const int* arpt, const int* acol, const double* aval,
                            const double* bval, int** crpt, int** ccol, double** cval, int M, int K, int N, int* cnnz,
                            brm_precise_timing* timing) {
     double ph[P_N] = {0}, tot = 0, h2d = 0, d2h_ = 0;
-    int st = host_entry<int>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, false, ph, &tot,
+    int st = host_entry<int>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, false,
+                             timing ? ph : nullptr, &tot,
                              &h2d, &d2h_);
     if (st == BRM_OK) fill_precise(timing, ph, tot, h2d, d2h_);
     dev_flush_deferred();
@@ -1512,7 +1524,8 @@ int brm_spgemm_upper_i32(const int* arpt, const int* acol, const double* aval, c
                          const double* bval, int** crpt, int** ccol, double** cval, int M, int K, int N, int* cnnz,
                          brm_upper_timing* timing) {
     double ph[P_N] = {0}, tot = 0, h2d = 0, d2h_ = 0;
-    int st = host_entry<int>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, true, ph, &tot,
+    int st = host_entry<int>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, true,
+                             timing ? ph : nullptr, &tot,
                              &h2d, &d2h_);
     if (st == BRM_OK) fill_upper(timing, ph, tot, h2d, d2h_);
     dev_flush_deferred();
@@ -1523,7 +1536,8 @@ int brm_spgemm_precise_i64(const int* arpt, const int* acol, const double* aval,
                            const double* bval, int64_t** crpt, int** ccol, double** cval, int M, int K, int N,
                            int64_t* cnnz, brm_precise_timing* timing) {
     double ph[P_N] = {0}, tot = 0, h2d = 0, d2h_ = 0;
-    int st = host_entry<int64_t>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, false, ph,
+    int st = host_entry<int64_t>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, false,
+                                 timing ? ph : nullptr,
                                  &tot, &h2d, &d2h_);
     if (st == BRM_OK) fill_precise(timing, ph, tot, h2d, d2h_);
     dev_flush_deferred();
@@ -1534,7 +1548,8 @@ int brm_spgemm_upper_i64(const int* arpt, const int* acol, const double* aval, c
                          const double* bval, int64_t** crpt, int** ccol, double** cval, int M, int K, int N,
                          int64_t* cnnz, brm_upper_timing* timing) {
     double ph[P_N] = {0}, tot = 0, h2d = 0, d2h_ = 0;
-    int st = host_entry<int64_t>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, true, ph,
+    int st = host_entry<int64_t>(arpt, acol, aval, brpt, bcol, bval, crpt, ccol, cval, M, K, N, cnnz, true,
+                                 timing ? ph : nullptr,
                                  &tot, &h2d, &d2h_);
     if (st == BRM_OK) fill_upper(timing, ph, tot, h2d, d2h_);
     dev_flush_deferred();

@@ -666,7 +666,7 @@ int brm_spgemm_batched_dev(const brm_pair* pairs, int npairs, int64_t** crpt, in
     const double t0 = now_s();
     double ph[P_N] = {0};
     DevOut out{};
-    int st = batched_run(pairs, npairs, (hipStream_t)stream, &out, row_off, ph);
+    int st = batched_run(pairs, npairs, (hipStream_t)stream, &out, row_off, timing ? ph : nullptr);
     if (st == BRM_OK) {
         *crpt = out.crpt;
         *ccol = out.ccol;

@@ -3,8 +3,8 @@
 // A product whose rows are all short (at most G = 64, or 32, lists and
 // products) spends more on the general pipeline's dozen launches and two
 // host round trips than on its kernels.  Such a product runs as:
-//   1. one fill clearing the state: flags, totals and the words through
-//      which the workgroups' places in C are handed on;
+//   1. one fill clearing the words through which the workgroups' places in C
+//      are handed on;
 //   2. k_small<G, P>: each workgroup takes a run of consecutive rows, in P
 //      passes of one row per group of G lanes.  The passes are batched stage
 //      by stage -- all row pointers, then all list descriptors, then all B
@@ -19,9 +19,10 @@
 //      per thread (row pointers, column range, sorted rows), as the general
 //      validation does.
 // C is allocated beforehand for G entries per row, a bound of nnz(C) when
-// every row is short.  The host reads the state once, at the end: a row with
-// more than G lists or products, or a B row with more than 64 entries, sets a
-// flag, and the product then goes through the general pipeline instead.
+// every row is short.  The scanning wavefront writes the totals and flags to
+// host memory, read once the stream has ended: a row with more than G lists or
+// products, or a B row with more than 64 entries, sets a flag, and the product
+// then goes through the general pipeline instead.
 #include <limits.h>
 
 #include <algorithm>
@@ -33,13 +34,14 @@
 namespace brm {
 namespace {
 
-// Two words per row workgroup, cleared beforehand: what it adds (own) and
-// what comes before it (pre).  The top bit marks a word as published; below
-// it products (from bit SC_IP) and nnz(C), both under 2^31.  Each word
-// carries its own value, so relaxed atomics (no cache invalidation or
-// write-back) are enough.
-constexpr int SC_IP = 31;
-constexpr uint64_t SC_SET = 1ull << 63, SC_LATE = 1ull << 62, SC_VAL = SC_LATE - 1ull;
+// One word per workgroup for what it adds (own) and, per row workgroup, one
+// for what comes before it (pre); cleared beforehand.  The top bit marks a
+// word as published; below it the flags, products (from bit SC_IP) and nnz(C).
+// Each word carries its own value, so relaxed atomics (no cache invalidation
+// or write-back) are enough.
+constexpr int SC_IP = 28, SC_FLAGS = 2 * SC_IP;
+constexpr uint64_t SC_SET = 1ull << 63, SC_LATE = 1ull << 62, SC_VAL = (1ull << SC_FLAGS) - 1ull;
+constexpr unsigned SC_BAD = 1u, SC_MISS = 2u;  // malformed operands; a row too long for this path
 static_assert((int64_t)SMALL_MAX_ROWS * BRM_WAVE < ((int64_t)1 << SC_IP), "two counts in a word");
 constexpr int SC_POLLS = 1 << 14;
 
@@ -61,32 +63,57 @@ __device__ __forceinline__ void sc_store(uint64_t* p, uint64_t v) {
 // it, so both waits are bounded: after SC_POLLS looks without a new word the
 // scanner marks the rest late, and the product is left to the general
 // pipeline.
-__device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nb) {
+// nrow words of row workgroups, then those of the others.
+__device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nrow, int n, SmallResult* res) {
     const int lane = lane_id();
     uint64_t sum = 0;
+    unsigned flags = 0;
     int polls = 0;
-    for (int base = 0; base < nb;) {
-        const uint64_t v = sc_load(&own[min(base + lane, nb - 1)]);
-        const uint64_t gap = __ballot((v & SC_SET) == 0 || base + lane >= nb);
+    for (int base = 0; base < n;) {
+        const uint64_t v = sc_load(&own[min(base + lane, n - 1)]);
+        const uint64_t gap = __ballot((v & SC_SET) == 0 || base + lane >= n);
         const int got = gap ? __ffsll((long long)gap) - 1 : BRM_WAVE;  // words up to the first unpublished one
         if (got == 0) {
             if (++polls <= SC_POLLS) continue;
-            for (int q = base + lane; q < nb; q += BRM_WAVE) sc_store(&pre[q], SC_SET | SC_LATE);
-            return;
+            for (int q = base + lane; q < nrow; q += BRM_WAVE) sc_store(&pre[q], SC_SET | SC_LATE);
+            flags |= SC_MISS;
+            break;
         }
         polls = 0;
         const uint64_t mine = lane < got ? v & SC_VAL : 0;
+        const unsigned f = lane < got ? (unsigned)(v >> SC_FLAGS) : 0u;
+        if (__ballot(f & SC_BAD)) flags |= SC_BAD;
+        if (__ballot(f & SC_MISS)) flags |= SC_MISS;
         const uint64_t inc = wave_incl_scan(mine);
-        if (lane < got) sc_store(&pre[base + lane], SC_SET | (sum + inc - mine));
+        if (lane < got && base + lane < nrow) sc_store(&pre[base + lane], SC_SET | (sum + inc - mine));
         sum += wave_last(inc);
         base += got;
     }
+    if (lane == 0) {
+        res->nnz = (int64_t)(sum & ((1ull << SC_IP) - 1ull));
+        res->ip = (int64_t)(sum >> SC_IP);
+        res->bad = (flags & SC_BAD) != 0;
+        res->miss = (flags & SC_MISS) != 0;
+        res->done = 1;
+    }
+}
+
+// The flags of the workgroup's threads, in every thread (fl: one word per
+// wavefront).
+template <int NW>
+__device__ unsigned block_flags(bool bad, bool miss, unsigned* fl) {
+    const unsigned mine = (__ballot(bad) != 0ull ? SC_BAD : 0u) | (__ballot(miss) != 0ull ? SC_MISS : 0u);
+    if (lane_id() == 0) fl[threadIdx.x / BRM_WAVE] = mine;
+    __syncthreads();
+    unsigned f = 0u;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) f |= fl[i];
+    return f;
 }
 
 // The prefix of workgroup b (called by one wavefront); 0 and *late when it
 // does not come.
-__device__ uint64_t await_prefix(uint64_t* own, const uint64_t* pre, int b, uint64_t mine, bool* late) {
-    if (lane_id() == 0) sc_store(&own[b], SC_SET | mine);
+__device__ uint64_t await_prefix(const uint64_t* pre, int b, bool* late) {
     for (int polls = 0; polls < 4 * SC_POLLS; ++polls) {
         const uint64_t v = sc_load(&pre[b]);
         if (v & SC_SET) {
@@ -123,16 +150,18 @@ struct SmallShape {
 template <int G, int P>
 __global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int nnzA, int nnzB, int row_blocks,
                                                               int64_t* __restrict__ crpt, int* __restrict__ ccol,
-                                                              double* __restrict__ cval, SmallState* __restrict__ st,
+                                                              double* __restrict__ cval, SmallResult* __restrict__ res,
                                                               uint64_t* __restrict__ own) {
     using S = SmallShape<G, P>;
     const int lane = lane_id();
     const int w = (int)(threadIdx.x / BRM_WAVE);
-    uint64_t* pre = own + row_blocks;
+    const int words = (int)gridDim.x - 1;
+    uint64_t* pre = own + words;
     if (blockIdx.x == 0) {
-        if (w == 0) scan_workgroups(own, pre, row_blocks);
+        if (w == 0) scan_workgroups(own, pre, row_blocks, words, res);
         return;
     }
+    __shared__ unsigned fl[S::WPB];
     const int b = (int)blockIdx.x - 1;
     if (b >= row_blocks) {
         // ---- B: one row per thread; entries 8 at a time (indices clamped
@@ -163,8 +192,8 @@ __global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int
         } else if (r == a.K) {
             bad = a.brpt[0] != 0 || a.brpt[a.K] != nnzB || a.arpt[0] != 0 || a.arpt[a.M] != nnzA;
         }
-        if (__ballot(bad) != 0ull && lane == 0) atomicOr(&st->err, (int)DERR_INVALID);
-        if (__ballot(lng) != 0ull && lane == 0) atomicOr(&st->miss, 1);
+        const unsigned f = block_flags<S::WPB>(bad, lng, fl);
+        if (threadIdx.x == 0) sc_store(&own[b], SC_SET | (uint64_t)f << SC_FLAGS);
         return;
     }
     __shared__ int rcnt[S::ROWS];      // nnz of the workgroup's rows
@@ -253,9 +282,7 @@ __global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int
             rip[p * S::RPP + slot] = ipn[p];
         }
     }
-    if (__ballot(bad) != 0ull && lane == 0) atomicOr(&st->err, (int)DERR_INVALID);
-    if (__ballot(miss) != 0ull && lane == 0) atomicOr(&st->miss, 1);
-    __syncthreads();
+    const unsigned flags = block_flags<S::WPB>(bad, miss, fl);
     // ---- the workgroup's rows in C: a scan over its rows, behind the
     // workgroups before it; C's row pointer from wavefront 0
     if (w == 0) {
@@ -269,8 +296,10 @@ __global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int
         const int64_t inc = wave_incl_scan(local);
         const int64_t agg = wave_last(inc);
         ips = wave_sum(ips);
+        if (lane == 0)
+            sc_store(&own[b], SC_SET | (uint64_t)flags << SC_FLAGS | (uint64_t)ips << SC_IP | (uint64_t)agg);
         bool late = false;
-        const uint64_t before = await_prefix(own, pre, b, ((uint64_t)ips << SC_IP) | (uint64_t)agg, &late);
+        const uint64_t before = await_prefix(pre, b, &late);
         const int64_t base = (int64_t)(before & ((1ull << SC_IP) - 1ull));
         int64_t off = base + inc - local;
 #pragma unroll
@@ -283,11 +312,7 @@ __global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int
             off += rcnt[k];
             if (row == a.M - 1) crpt[a.M] = off;
         }
-        if (lane == 0 && late) atomicOr(&st->miss, 1);
-        if (lane == 0 && b == row_blocks - 1) {
-            st->nnz = base + agg;
-            st->ip = (int64_t)(before >> SC_IP) + ips;
-        }
+        if (lane == 0 && late) res->late = 1;
     }
     __syncthreads();
 #pragma unroll
@@ -305,15 +330,22 @@ int64_t row_blocks_of(int M) {
     return ((int64_t)M + SmallShape<G, P>::ROWS - 1) / SmallShape<G, P>::ROWS;
 }
 
+// the K rows of B and the ends of the row pointers
+template <int G>
+int64_t b_blocks_of(int K) {
+    constexpr int NT = SmallShape<G, 1>::NT;
+    return ((int64_t)K + 1 + NT - 1) / NT;
+}
+
 template <int G, int P>
 hipError_t launch_small_gp(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
-                           SmallState* st, uint64_t* own, hipStream_t s) {
+                           SmallResult* res, uint64_t* own, hipStream_t s) {
     using S = SmallShape<G, P>;
     const int64_t rb = row_blocks_of<G, P>(a.M);
-    const int64_t bb = ((int64_t)a.K + 1 + S::NT - 1) / S::NT;
+    const int64_t bb = b_blocks_of<G>(a.K);
     if (1 + rb + bb > INT32_MAX || nnzA > INT32_MAX || nnzB > INT32_MAX) return hipErrorInvalidValue;
     ProfScope ps_("k_small", s);
-    k_small<G, P><<<(unsigned)(1 + rb + bb), S::NT, 0, s>>>(a, (int)nnzA, (int)nnzB, (int)rb, crpt, ccol, cval, st, own);
+    k_small<G, P><<<(unsigned)(1 + rb + bb), S::NT, 0, s>>>(a, (int)nnzA, (int)nnzB, (int)rb, crpt, ccol, cval, res, own);
     return hipGetLastError();
 }
 
@@ -332,34 +364,32 @@ int passes_of(int M) {
 
 template <int G>
 hipError_t launch_small_g(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
-                          SmallState* st, uint64_t* own, hipStream_t s) {
+                          SmallResult* res, uint64_t* own, hipStream_t s) {
     switch (passes_of<G>(a.M)) {
-        case 1: return launch_small_gp<G, 1>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
-        case 2: return launch_small_gp<G, 2>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
-        default: return launch_small_gp<G, SM_P>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
+        case 1: return launch_small_gp<G, 1>(a, nnzA, nnzB, crpt, ccol, cval, res, own, s);
+        case 2: return launch_small_gp<G, 2>(a, nnzA, nnzB, crpt, ccol, cval, res, own, s);
+        default: return launch_small_gp<G, SM_P>(a, nnzA, nnzB, crpt, ccol, cval, res, own, s);
     }
 }
 
 template <int G>
-int64_t states_of(int M) {
+int64_t words_of(int M, int K) {
     const int p = passes_of<G>(M);
-    return p == 1 ? row_blocks_of<G, 1>(M) : p == 2 ? row_blocks_of<G, 2>(M) : row_blocks_of<G, SM_P>(M);
+    const int64_t rb = p == 1 ? row_blocks_of<G, 1>(M) : p == 2 ? row_blocks_of<G, 2>(M) : row_blocks_of<G, SM_P>(M);
+    return 2 * rb + b_blocks_of<G>(K);
 }
 
 }  // namespace
 
-int64_t small_state_words(int M, int group) {
-    return (int64_t)(sizeof(SmallState) / 8) + 2 * (group == 32 ? states_of<32>(M) : states_of<64>(M));
-}
+int64_t small_words(int M, int K, int group) { return group == 32 ? words_of<32>(M, K) : words_of<64>(M, K); }
 
 hipError_t launch_small(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
-                        SmallState* st, int group, hipStream_t s) {
+                        SmallResult* res, uint64_t* words, int group, hipStream_t s) {
     if (a.M < 1 || a.K < 1 || nnzA < 1 || nnzB < 1) return hipErrorInvalidValue;
-    hipError_t e = launch_fill_i64((int64_t*)st, small_state_words(a.M, group), 0, s);
+    hipError_t e = launch_fill_i64((int64_t*)words, small_words(a.M, a.K, group), 0, s);
     if (e != hipSuccess) return e;
-    uint64_t* own = reinterpret_cast<uint64_t*>(st) + sizeof(SmallState) / 8;
-    return group == 32 ? launch_small_g<32>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s)
-                       : launch_small_g<64>(a, nnzA, nnzB, crpt, ccol, cval, st, own, s);
+    return group == 32 ? launch_small_g<32>(a, nnzA, nnzB, crpt, ccol, cval, res, words, s)
+                       : launch_small_g<64>(a, nnzA, nnzB, crpt, ccol, cval, res, words, s);
 }
 
 }  // namespace brm
