@@ -384,9 +384,11 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
     tr.mark("long info read back");
     // ---- partition into waves and size every buffer for the largest wave
     struct Wave {
-        int k0, k1;
+        int k0, k1, passes;
+        int64_t nroots[MAX_PASSES + 1];
+        std::vector<int> large;
         int64_t ws_tot[2], sl_tot, tab_tot, leaf_cap, child_cap;
-        std::vector<int64_t> wsb, slb, tabb, seg;  // wsb: two per row (buffers 0 and 1)
+        std::vector<int64_t> wsb, slb, tabb, chb, root, seg;  // wsb: two per row (buffers 0 and 1)
     };
     std::vector<Wave> waves;
     int64_t mx_ws[2] = {0, 0}, mx_sl = 0, mx_leaf = 0, mx_child = 0, mx_task = 0, mx_tab = 0;
@@ -406,6 +408,10 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         w.wsb.resize(2 * (size_t)(k1 - k0));
         w.slb.resize(k1 - k0);
         w.tabb.resize(k1 - k0);
+        w.chb.resize(k1 - k0);
+        w.root.resize(k1 - k0);
+        std::fill(std::begin(w.nroots), std::end(w.nroots), 0);
+        w.passes = 0;
         std::vector<int64_t> capP(MAX_PASSES + 1, 0);
         for (int k = 0; k < k1 - k0; ++k) {
             const int Lr = len[k0 + k];
@@ -423,6 +429,10 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
             w.ws_tot[0] += ws_need(k0 + k, 0);
             w.ws_tot[1] += ws_need(k0 + k, 1);
             w.sl_tot += (int64_t)2 << H;
+            w.passes = std::max(w.passes, J);
+            w.chb[k] = w.child_cap;
+            w.root[k] = ip[k0 + k] > 0 ? w.nroots[J]++ : -1;
+            if (Lr > BRM_WAVE) w.large.push_back(k);
             w.leaf_cap += Lr;
             w.child_cap += 2 * (int64_t)Lr + 2;
             for (int j = 1; j <= J; ++j) capP[j] += (int64_t)(Lr >> std::min(j * pass_bits, H)) + 2;
@@ -488,10 +498,10 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
     // not hold the sort's buffers).
     struct WaveTables {
         int* rows_w = nullptr;
-        int64_t *wsb_d = nullptr, *slb_d = nullptr, *tabb_d = nullptr, *seg_d = nullptr, *slots = nullptr, *counters = nullptr;
+        int64_t *wsb_d = nullptr, *slb_d = nullptr, *tabb_d = nullptr, *chb_d = nullptr, *root_d = nullptr, *seg_d = nullptr, *slots = nullptr, *counters = nullptr;
         GroupTask* tasks = nullptr;
         Child* children = nullptr;
-        int* node_tab = nullptr;
+        int *node_tab = nullptr, *large_d = nullptr;
         uint32_t *tkey = nullptr, *tkey_out = nullptr;
         int *tidx_in = nullptr, *tidx_out = nullptr;
         unsigned char* ttmp = nullptr;
@@ -505,12 +515,18 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
     // pass, the roots of its heaviest rows, then runs beside wave w+1's
     // planning and first pass.
     const bool overlap = bitmap && arena < 0 && ttmp_bytes > 0 && waves.size() > 1 && thread_side_streams();
+    const bool placed = bitmap && arena < 0;  // child and root entries
     WaveTables wt[2];
     for (int par = 0; par < (overlap ? 2 : 1); ++par) {
         WaveTables& t = wt[par];
         BRMC(wsc.alloc(&t.rows_w, mx_rows, "wave rows"));
         BRMC(wsc.alloc(&t.wsb_d, 2 * (int64_t)mx_rows, "wave ws_base"));
         BRMC(wsc.alloc(&t.slb_d, mx_rows, "wave slot_base"));
+        if (placed) {
+            BRMC(wsc.alloc(&t.chb_d, mx_rows, "wave child_base"));
+            BRMC(wsc.alloc(&t.root_d, mx_rows, "wave root_task"));
+            BRMC(wsc.alloc(&t.large_d, mx_rows, "wave large rows"));
+        }
         if (nb > 0) {
             BRMC(wsc.alloc(&t.tabb_d, mx_rows, "wave tab_base"));
             BRMC(wsc.alloc(&t.node_tab, mx_tab, "node block table"));
@@ -600,6 +616,12 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         HIPC(hipMemcpyAsync(t.slb_d, w.slb.data(), sizeof(int64_t) * nw, hipMemcpyHostToDevice, ws));
         if (nb > 0)
             HIPC(hipMemcpyAsync(t.tabb_d, w.tabb.data(), sizeof(int64_t) * nw, hipMemcpyHostToDevice, ws));
+        if (placed) {
+            HIPC(hipMemcpyAsync(t.chb_d, w.chb.data(), sizeof(int64_t) * nw, hipMemcpyHostToDevice, ws));
+            HIPC(hipMemcpyAsync(t.root_d, w.root.data(), sizeof(int64_t) * nw, hipMemcpyHostToDevice, ws));
+            if (!w.large.empty())
+                HIPC(hipMemcpyAsync(t.large_d, w.large.data(), sizeof(int) * w.large.size(), hipMemcpyHostToDevice, ws));
+        }
         HIPC(hipMemcpyAsync(t.seg_d, w.seg.data(), sizeof(int64_t) * (MAX_PASSES + 2), hipMemcpyHostToDevice, ws));
         HIPC(launch_fill_i64(t.counters, CNT_N, 0, ws));
         HIPC(launch_fill_i64(t.slots, w.sl_tot, 0, ws));
@@ -610,6 +632,11 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         la.ws_base = t.wsb_d;
         la.slot_base = t.slb_d;
         la.tab_base = t.tabb_d;
+        la.child_base = t.chb_d;
+        la.root_task = t.root_d;
+        la.large = t.large_d;
+        la.nlarge = (int)w.large.size();
+        for (int j = 0; j <= MAX_PASSES; ++j) la.nroots[j] = placed ? w.nroots[j] : 0;
         la.arpt = a.arpt;
         la.acol = a.acol;
         la.aval = a.aval;
@@ -637,7 +664,9 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
 
         HIPC(launch_leaf(leaves, cnt[CNT_LEAF], a, wcol, wval, t.slots, t.counters, o, ws));
         tr.mark("leaves", cnt[CNT_LEAF]);
-        const int passes = (int)cnt[CNT_MAXP];
+        const int passes = w.passes;
+        if (placed)  // the counters hold the tasks below the roots
+            for (int j = 0; j <= MAX_PASSES; ++j) cnt[CNT_TASK0 + j] += w.nroots[j];
         // the last pass that reads or writes buffer 1: passes j writing
         // nodes below the root into buffer j & 1, reading buffer (j-1) & 1
         int b1_last = 0;

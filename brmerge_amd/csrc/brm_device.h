@@ -74,6 +74,13 @@ __device__ __forceinline__ T wave_sum(T x) {
     return wave_last(wave_incl_scan(x));
 }
 
+// x of lane l (uniform).
+__device__ __forceinline__ int64_t readlane64(int64_t x, int l) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)x, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)x >> 32), l);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 // ---------------------------------------------------------------- block scans
 // Exclusive scan over the block; returns this thread's exclusive prefix and
 // the block total in *total.  `sm` must hold NT/64 + 1 elements of T.

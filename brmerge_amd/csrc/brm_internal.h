@@ -114,7 +114,6 @@ struct LeafTask {
 
 // Counters written by the planner and the merge kernels.
 constexpr int CNT_LEAF = 0;      // leaf tasks
-constexpr int CNT_MAXP = 1;      // passes needed by the wave
 constexpr int CNT_LEAF_IP = 2;   // products inside leaves
 constexpr int CNT_LEAF_OUT = 3;  // leaf output elements
 constexpr int CNT_GRP_IN = 4;    // group merge input elements
@@ -132,6 +131,15 @@ struct LongArgs {
     const int64_t* ws_base;  // per row: [2] element offsets into workspace buffers 0 and 1
     const int64_t* slot_base;
     const int64_t* tab_base;  // per row: its first row of the node table, or nullptr
+    // Entries placed beforehand, or nullptr (all by counters): per row its
+    // first child entry (2 per list and 2 more each), and its root among the
+    // nroots[j] first tasks of its last pass j (-1: no products); and the
+    // nlarge rows of more than 64 lists.
+    const int64_t* child_base;
+    const int64_t* root_task;
+    const int* large;
+    int nlarge;
+    int64_t nroots[MAX_PASSES + 1];
     const int* arpt;
     const int* acol;
     const double* aval;

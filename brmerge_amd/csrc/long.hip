@@ -182,19 +182,34 @@ __device__ void emit_group(const LongArgs& la, int row, int a0, const int64_t* i
 
 // Without a frontier (frontier_cap 0: every non-empty list is a child in
 // place) the children of pass-j node (s, h_j) are exactly the non-empty
-// nodes at height h_{j-1} inside it, at most PL_NT of them: the workgroup
-// emits each node's children together, thread t taking child slot t, with
-// a block scan for their order.
-// Nodes of fan-in F = 2^(hj - hp) <= 2^pass_bits: the workgroup plans
-// PL_NT / F nodes per step, one child slot per thread, with one scan and one
-// reservation of child entries for all of them.
+// nodes at height h_{j-1} inside it.  Nodes of fan-in F = 2^(hj - hp) <=
+// 2^pass_bits: the workgroup plans PL_NT / F nodes per step, one child slot
+// per thread, with one scan for the order of their children and tasks.
+//
+// Where entries go: with `chb` (the row's first child entry) and `root` (the
+// row's root among the roots of its pass) every step has its own place for
+// children, one entry per slot, and steps y0, y0 + dy, ... are planned; only the
+// tasks below the root come from a counter, one atomic per step.  Without them
+// (-1) children, and all tasks, come from counters.
+__device__ void put_task(const LongArgs& la, int j, int64_t idx, const GroupTask& T, int64_t ip, int* err) {
+    if (idx >= la.task_seg[j + 1] - la.task_seg[j]) {
+        atomicOr(err, (int)DERR_CAPACITY);
+        return;
+    }
+    la.tasks[la.task_seg[j] + idx] = T;
+    if (la.task_key) la.task_key[la.task_seg[j] + idx] = (uint32_t)min(ip, (int64_t)UINT32_MAX);
+}
+
 __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int64_t* ipr, int L, int H, int J,
-                                 WsBase wsb, int64_t slb, int64_t tabb, int64_t final_off, int* err) {
+                                 WsBase wsb, int64_t slb, int64_t tabb, int64_t chb, int64_t root_at, int y0, int dy,
+                                 int64_t final_off, int* err) {
     __shared__ int64_t sm[PL_NT / BRM_WAVE + 1];
-    __shared__ int64_t cbase;
-    __shared__ int64_t lead[PL_NT + 1];  // child prefix at each node's first slot; [G]: the step's total
+    __shared__ int64_t cbase, tbase;
+    __shared__ int lead[PL_NT + 1];  // child prefix at each node's first slot; [G]: the step's total
     const int t = threadIdx.x;
     const int pb = la.pass_bits;
+    int64_t slots = 0;  // child slots of the passes before
+    int step = 0;
     for (int j = 1; j <= J; ++j) {
         const int hj = pass_height(j, H, pb);
         const int hp = j == 1 ? 0 : pass_height(j - 1, H, pb);
@@ -204,7 +219,8 @@ __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int6
         const int G = PL_NT >> fb;   // nodes per step
         const int k = t >> fb;       // this thread's node in the step
         const int c = t & ((1 << fb) - 1);
-        for (int nd0 = 0; nd0 < nnodes; nd0 += G) {
+        for (int nd0 = 0; nd0 < nnodes; nd0 += G, ++step) {
+            if (step % dy != y0) continue;  // uniform
             const int nd = nd0 + k;
             bool live = false;
             int s = 0, e = 0;
@@ -218,16 +234,18 @@ __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int6
             Src src{};
             src.kind = SRC_EMPTY;
             if (live && q < e) src = make_src(la, a0, ipr, L, H, q, hp, (j - 1) & 1, wsb, slb);
-            const int64_t has = src.kind != SRC_EMPTY ? 1 : 0;
-            int64_t nc;
-            const int64_t rank = block_excl_scan<PL_NT>(has, sm, &nc);
+            const bool has = src.kind != SRC_EMPTY, task = c == 0 && live;
+            int64_t all;  // children in the low half, tasks in the high half
+            const int64_t pre = block_excl_scan<PL_NT>((int64_t)has | (int64_t)task << 32, sm, &all);
+            const int rank = (int)(uint32_t)pre, nc = (int)(uint32_t)all, nt = (int)(all >> 32);
             if (c == 0) lead[k] = rank;
             if (t == 0) {
                 lead[G] = nc;
-                const unsigned long long cb =
-                    atomicAdd((unsigned long long*)&la.counters[CNT_CHILD], (unsigned long long)nc);
-                cbase = (int64_t)cb;
-                if ((int64_t)cb + nc > la.child_cap) atomicOr(err, (int)DERR_CAPACITY);
+                cbase = chb >= 0 ? chb + slots + ((int64_t)nd0 << fb)
+                                 : (int64_t)atomicAdd((unsigned long long*)&la.counters[CNT_CHILD], (unsigned long long)nc);
+                if (root && root_at >= 0) tbase = root_at;
+                else if (nt) tbase = la.nroots[j] + (int64_t)atomicAdd((unsigned long long*)&la.counters[CNT_TASK0 + j], (unsigned long long)nt);
+                if (cbase + nc > la.child_cap) atomicOr(err, (int)DERR_CAPACITY);
             }
             __syncthreads();
             const int64_t cb = cbase;
@@ -242,7 +260,7 @@ __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int6
                                                     : 0;
                     la.children[cb + rank] = ch;
                 }
-                if (c == 0 && live) {
+                if (task) {
                     GroupTask T;
                     T.row = row;
                     T.nchild = (int)(lead[k + 1] - lead[k]);
@@ -260,23 +278,82 @@ __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int6
                         T.slot = slb + heap_idx(H, s, hj);
                         T.tab = tabb >= 0 ? node_tab(tabb, L, H, pb, j, s) : -1;
                     }
-                    const unsigned long long idx =
-                        atomicAdd((unsigned long long*)&la.counters[CNT_TASK0 + j], 1ull);
-                    if ((int64_t)idx >= la.task_seg[j + 1] - la.task_seg[j]) {
-                        atomicOr(err, (int)DERR_CAPACITY);
-                    } else {
-                        la.tasks[la.task_seg[j] + (int64_t)idx] = T;
-                        if (la.task_key)
-                            la.task_key[la.task_seg[j] + (int64_t)idx] =
-                                (uint32_t)min(ipr[e] - ipr[s], (int64_t)UINT32_MAX);
-                    }
+                    put_task(la, j, tbase + (int)(pre >> 32), T, ipr[e] - ipr[s], err);
                 }
             }
             __syncthreads();  // cbase and lead are rewritten by the next step
         }
+        slots += ((L - 1) >> hp) + 1;
     }
 }
 
+// Planning without counters where places are known beforehand.  An atomic on
+// one counter takes some 8 ns whoever issues it, so that a workgroup per row
+// with three of them bounded the planning: 2,160 us for 68,825 rows (120,795
+// tasks) of an R-MAT product of 2^18 rows, now 486; 133 us at 2^14 rows, now 35.
+// (Eight rows per workgroup with one atomic, larger rows one after the other:
+// 1,720 and 218 us; two or eight workgroups per larger row: as four, to 1 %.)
+//
+// Rows of at most 64 lists without a frontier, a wavefront each: the root over
+// the row's non-empty lists.
+__global__ __launch_bounds__(PL_NT) void k_plan_small(LongArgs la, int r0, int nr, int* err) {
+    const int r = r0 + blockIdx.x * (PL_NT / BRM_WAVE) + threadIdx.x / BRM_WAVE;
+    if (r >= r0 + nr) return;
+    const int row = la.rows[r], a0 = la.arpt[row], L = la.arpt[row + 1] - a0;
+    const int64_t root_at = la.root_task[r], chb = la.child_base[r];
+    if (L > BRM_WAVE || root_at < 0) return;
+    const int lane = lane_id();
+    const int64_t* ipr = la.ipA + a0;
+    const int64_t p0 = ipr[min(lane, L)], p1 = ipr[min(lane + 1, L)];
+    const uint64_t full = __ballot(p1 > p0);
+    const int nc = __popcll(full);
+    if (chb + nc > la.child_cap) {
+        if (lane == 0) atomicOr(err, (int)DERR_CAPACITY);
+        return;
+    }
+    if (p1 > p0) {
+        const int c = la.acol[a0 + lane];
+        Child ch;
+        ch.src = Src{};
+        ch.src.kind = SRC_VIRTUAL;
+        ch.src.off = la.brpt[c];
+        ch.src.len = p1 - p0;
+        ch.src.scale = la.aval[a0 + lane];
+        ch.lid = lane;
+        ch.tab = c;  // the B row
+        la.children[chb + __builtin_amdgcn_mbcnt_hi((unsigned)(full >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((unsigned)full, 0u))] = ch;
+    }
+    if (lane == 0) {
+        GroupTask T;
+        T.row = row;
+        T.nchild = nc;
+        T.cbase = chb;
+        T.final_dst = 1;
+        T.dst_buf = 0;
+        T.dst_off = la.final_off ? la.final_off[row] : ipr[0];
+        T.slot = -1;
+        T.tab = -1;
+        put_task(la, 1, root_at, T, ipr[L] - ipr[0], err);
+    }
+}
+static_assert(BPASS_BITS == 6, "a node of one list per lane");
+
+// Rows of more lists, PL_Y workgroups each.
+constexpr int PL_Y = 4;
+__global__ __launch_bounds__(PL_NT) void k_plan_large(LongArgs la, const int* __restrict__ large, int n0, int* err) {
+    const int r = large[n0 + blockIdx.x / PL_Y];
+    const int row = la.rows[r], a0 = la.arpt[row], L = la.arpt[row + 1] - a0;
+    const int64_t* ipr = la.ipA + a0;
+    const int H = ceil_log2i(L), pb = la.pass_bits, J = (H + pb - 1) / pb;
+    const WsBase wsb{la.ws_base[2 * (int64_t)r], la.ws_base[2 * (int64_t)r + 1]};
+    plan_no_frontier(la, row, a0, ipr, L, H, J, wsb, la.slot_base[r], la.tab_base ? la.tab_base[r] : -1,
+                     la.child_base[r], la.root_task[r], blockIdx.x % PL_Y, PL_Y,
+                     la.final_off ? la.final_off[row] : ipr[0], err);
+}
+
+// A workgroup per row: rows with a frontier, and the fixed-buffer arena,
+// whose budget does not hold the places of k_plan_small and k_plan_large.
 __global__ __launch_bounds__(PL_NT) void k_plan(LongArgs la, int r0, int* err) {
     const Fit cap{la.frontier_cap, la.lmax, la.log_lmax};
     const int r = r0 + blockIdx.x;
@@ -291,8 +368,8 @@ __global__ __launch_bounds__(PL_NT) void k_plan(LongArgs la, int r0, int* err) {
     const int64_t slb = la.slot_base[r];
     const int64_t final_off = la.final_off ? la.final_off[row] : ipr[0];
     if (la.frontier_cap == 0 && (1 << pb) <= PL_NT) {
-        plan_no_frontier(la, row, a0, ipr, L, H, J, wsb, slb, la.tab_base ? la.tab_base[r] : -1, final_off, err);
-        if (threadIdx.x == 0) atomicMax((unsigned long long*)&la.counters[CNT_MAXP], (unsigned long long)J);
+        plan_no_frontier(la, row, a0, ipr, L, H, J, wsb, slb, la.tab_base ? la.tab_base[r] : -1, -1, -1, 0, 1, final_off,
+                         err);
         return;
     }
 
@@ -344,7 +421,6 @@ __global__ __launch_bounds__(PL_NT) void k_plan(LongArgs la, int r0, int* err) {
             emit_group(la, row, a0, ipr, L, H, j, s, hj, pass_height(j - 1, H, pb), cap, wsb, slb, final_off, err);
         }
     }
-    if (threadIdx.x == 0) atomicMax((unsigned long long*)&la.counters[CNT_MAXP], (unsigned long long)J);
 }
 
 // ---------------------------------------------------------------- group merge
@@ -572,9 +648,23 @@ hipError_t launch_plan(const LongArgs& la, int* err, hipStream_t s) {
     if (la.nrows <= 0) return hipSuccess;
     {
         ProfScope ps_("k_plan", s);
-        const int64_t ch = launch_chunk(PL_NT);
-        for (int64_t b = 0; b < la.nrows; b += ch)
-            k_plan<<<(unsigned)std::min<int64_t>(ch, la.nrows - b), PL_NT, 0, s>>>(la, (int)b, err);
+        if (la.root_task) {
+            if (la.frontier_cap != 0 || la.pass_bits != BPASS_BITS) return hipErrorInvalidValue;
+            int64_t ch = launch_chunk(BRM_WAVE);
+            for (int64_t b = 0; b < la.nrows; b += ch) {
+                const int c = (int)std::min<int64_t>(ch, la.nrows - b);
+                constexpr int W = PL_NT / BRM_WAVE;
+                k_plan_small<<<(unsigned)((c + W - 1) / W), PL_NT, 0, s>>>(la, (int)b, c, err);
+            }
+            ch = launch_chunk(PL_NT * PL_Y);
+            for (int64_t b = 0; b < la.nlarge; b += ch)
+                k_plan_large<<<(unsigned)(std::min<int64_t>(ch, la.nlarge - b) * PL_Y), PL_NT, 0, s>>>(la, la.large,
+                                                                                                       (int)b, err);
+        } else {
+            const int64_t ch = launch_chunk(PL_NT);
+            for (int64_t b = 0; b < la.nrows; b += ch)
+                k_plan<<<(unsigned)std::min<int64_t>(ch, la.nrows - b), PL_NT, 0, s>>>(la, (int)b, err);
+        }
     }
     return hipGetLastError();
 }

@@ -198,12 +198,6 @@ __device__ __forceinline__ RmRows rm_rows(const int* __restrict__ rows, int nrow
     return w;
 }
 
-__device__ __forceinline__ int64_t readlane64(int64_t x, int l) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)x, l);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)x >> 32), l);
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
 // One row's lists, one per lane: B row range and A value.  Fetched in two
 // dependent steps while the row before is worked on.
 struct RmList {
