@@ -218,14 +218,18 @@ __global__ __launch_bounds__(HS_NT) void k_sym_hash(const int* __restrict__ rows
 }
 
 // Long rows: distinct columns counted with an LDS bitmap of up to 2^20
-// columns per pass (128 KB); wider matrices take several column passes.
+// columns per pass (128 KB); wider matrices take several column passes.  The
+// bitmap is as large as B's columns need, so that up to 2^18 of them leave
+// room for a second workgroup on the CU, to load while the first waits at a
+// barrier (R-MAT of 2^18 rows: 4,013 us with 128 KB for all, now 2,538; 2^14
+// rows: 125 and 70).  Workgroups of 512 threads take 2,365 and 114, of 256
+// 2,697 and 200: the last hub rows run alone.
 // Lists are taken in chunks of BM_CHUNK: their product offsets and B row
 // starts go to LDS first, so a product's column is one global load, and
 // each thread handles BM_U consecutive products per step with their loads
 // issued together.
 constexpr int BM_NT = 1024;
 constexpr int BM_BITS = 1 << 20;
-constexpr int BM_WORDS = BM_BITS / 32;
 constexpr int BM_CHUNK = 2048;
 constexpr int BM_U = 8;
 
@@ -246,19 +250,20 @@ __device__ __forceinline__ int sym_chunk_lists(const int64_t* __restrict__ ipA, 
     return lo;
 }
 
+// bits: columns of a pass
 __global__ __launch_bounds__(BM_NT) void k_sym_bitmap(const int* __restrict__ rows, int nrows, RowArgs a,
-                                                      int64_t* __restrict__ nnzrow, int64_t pcap) {
+                                                      int64_t* __restrict__ nnzrow, int64_t pcap, int bits) {
     extern __shared__ __align__(16) unsigned char smraw[];
     unsigned* bm = reinterpret_cast<unsigned*>(smraw);
-    int* loff = reinterpret_cast<int*>(smraw + sizeof(unsigned) * BM_WORDS);
+    int* loff = reinterpret_cast<int*>(smraw + bits / 8);
     int* bst = loff + BM_CHUNK + 8;
     int64_t* red = reinterpret_cast<int64_t*>(bst + BM_CHUNK + 8);
     const int t = threadIdx.x;
     const int row = rows[blockIdx.x];
     const int ab = a.arpt[row], ae = a.arpt[row + 1];
     int64_t total = 0;
-    for (int64_t c0 = 0; c0 < a.N; c0 += BM_BITS) {
-        const int64_t span = min((int64_t)BM_BITS, (int64_t)a.N - c0);
+    for (int64_t c0 = 0; c0 < a.N; c0 += bits) {
+        const int64_t span = min((int64_t)bits, (int64_t)a.N - c0);
         const int words = (int)((span + 31) / 32);
         const int c0i = (int)c0;
         const unsigned span32 = (unsigned)span;
@@ -313,10 +318,10 @@ __global__ __launch_bounds__(BM_NT) void k_sym_bitmap(const int* __restrict__ ro
     if (t == 0) nnzrow[row] = total;
 }
 
-constexpr size_t bitmap_smem() {
-    return sizeof(unsigned) * BM_WORDS + 2 * sizeof(int) * (BM_CHUNK + 8) + sizeof(int64_t) * (BM_NT / BRM_WAVE + 2);
+constexpr size_t bitmap_smem(int bits) {
+    return bits / 8 + 2 * sizeof(int) * (BM_CHUNK + 8) + sizeof(int64_t) * (BM_NT / BRM_WAVE + 2);
 }
-static_assert(bitmap_smem() <= 160 * 1024, "LDS of one CU");
+static_assert(bitmap_smem(BM_BITS) <= 160 * 1024, "LDS of one CU");
 
 template <int NT, int CAP, int LMAX>
 hipError_t medium_numeric_t(const int* rows, int n, const RowArgs& a, const OutArgs& o, hipStream_t s,
@@ -439,13 +444,15 @@ hipError_t launch_hash_count(const int* rows, int n, const RowArgs& a, int64_t* 
 hipError_t launch_long_count(const int* rows, int n, const RowArgs& a, int64_t* nnzrow, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     static SmemLimit lim;
-    if (hipError_t e = lim.raise((const void*)k_sym_bitmap, (int)bitmap_smem()); e != hipSuccess) return e;
+    if (hipError_t e = lim.raise((const void*)k_sym_bitmap, (int)bitmap_smem(BM_BITS)); e != hipSuccess) return e;
+    const int bits = (int)std::min<int64_t>(((int64_t)a.N + 1023) / 1024 * 1024, BM_BITS);  // 128-byte steps
     {
         ProfScope ps_("k_sym_bitmap", s);
         const int64_t ch = launch_chunk(BM_NT);
         for (int64_t b = 0; b < n; b += ch) {
             const int c = (int)std::min<int64_t>(ch, n - b);
-            k_sym_bitmap<<<c, BM_NT, bitmap_smem(), s>>>(rows + b, c, a, nnzrow, params().sym_chunk_products);
+            k_sym_bitmap<<<c, BM_NT, bitmap_smem(bits), s>>>(rows + b, c, a, nnzrow, params().sym_chunk_products,
+                                                        bits);
         }
     }
     return hipGetLastError();
