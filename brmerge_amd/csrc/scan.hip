@@ -195,7 +195,7 @@ hipError_t scan_impl(F f, int64_t n, int64_t* out, hipStream_t s) {
 // scan is spread over the chip (26 scans of a served batch's 20 requests: 846 us
 // in tiles of 4,096, now 357 us), else of 2,048 (of 4,096 a thread's elements
 // take 98 registers and a batch of 192 products 20 us more).  In the
-// fixed-buffer arena 2,048 always: fewer tile totals.
+// fixed-buffer arena 4,096 always: the tile totals take its room.
 template <typename F>
 hipError_t scan(F f, int64_t n, int64_t* out, hipStream_t s) {
     if (n <= 0) {
@@ -203,7 +203,8 @@ hipError_t scan(F f, int64_t n, int64_t* out, hipStream_t s) {
         k_zero1<<<1, 1, 0, s>>>(out);
         return hipGetLastError();
     }
-    return n <= 512 * 4 * SCAN_NT && arena_remaining() < 0 ? scan_impl<F, 4>(f, n, out, s) : scan_impl<F, 8>(f, n, out, s);
+    if (arena_remaining() >= 0) return scan_impl<F, 16>(f, n, out, s);
+    return n <= 512 * 4 * SCAN_NT ? scan_impl<F, 4>(f, n, out, s) : scan_impl<F, 8>(f, n, out, s);
 }
 
 }  // namespace
