@@ -20,8 +20,9 @@
 // the bucket counters hold one 16-bit count per wavefront, so that a bucket
 // fills nearly in list order, elements being numbered child by child.
 //
-// What bounds it: LDS instructions and the barriers of a round (HBM traffic
-// is a tenth of the peak).  Hence 2,048 elements a round in under 40 KB, four
+// What bounds it: LDS instructions and the barriers of a round, while B stays
+// in the caches (R-MAT of 2^18 rows); at 2^20 rows also HBM, 3.8 TB/s of it
+// where a copy reaches 4.6.  Hence 2,048 elements a round in under 40 KB, four
 // workgroups per CU (three: 44.4 ms against 38.9 on R-MAT, 2^18 rows); the
 // next round's loads in flight over this round's sums, and the plan of the
 // round after it by wavefront 0 while the others sum (37.6 ms to 35.2; it had
