@@ -1,4 +1,7 @@
-// Bitmap-rank group merge for long rows (group_cfg 4).
+// Bitmap-rank group merge for long rows (group_cfg 4) without tables: in the
+// fixed-buffer arena, and where the column tiles' tables would not pay or do
+// not fit (btile.hip has the engine with them, which takes about half the time
+// per product).
 //
 // One workgroup materialises one tree node above the lists of a long row
 // from up to BGROUP_KMAX child lists (B rows read in place, or nodes of the previous

@@ -180,6 +180,16 @@ __device__ void emit_group(const LongArgs& la, int row, int a0, const int64_t* i
     la.tasks[la.task_seg[j] + (int64_t)idx] = T;
 }
 
+// Task number idx of pass j, over ip products.
+__device__ void put_task(const LongArgs& la, int j, int64_t idx, const GroupTask& T, int64_t ip, int* err) {
+    if (idx >= la.task_seg[j + 1] - la.task_seg[j]) {
+        atomicOr(err, (int)DERR_CAPACITY);
+        return;
+    }
+    la.tasks[la.task_seg[j] + idx] = T;
+    if (la.task_key) la.task_key[la.task_seg[j] + idx] = (uint32_t)min(ip, (int64_t)UINT32_MAX);
+}
+
 // Without a frontier (frontier_cap 0: every non-empty list is a child in
 // place) the children of pass-j node (s, h_j) are exactly the non-empty
 // nodes at height h_{j-1} inside it.  Nodes of fan-in F = 2^(hj - hp) <=
@@ -191,15 +201,6 @@ __device__ void emit_group(const LongArgs& la, int row, int a0, const int64_t* i
 // children, one entry per slot, and steps y0, y0 + dy, ... are planned; only the
 // tasks below the root come from a counter, one atomic per step.  Without them
 // (-1) children, and all tasks, come from counters.
-__device__ void put_task(const LongArgs& la, int j, int64_t idx, const GroupTask& T, int64_t ip, int* err) {
-    if (idx >= la.task_seg[j + 1] - la.task_seg[j]) {
-        atomicOr(err, (int)DERR_CAPACITY);
-        return;
-    }
-    la.tasks[la.task_seg[j] + idx] = T;
-    if (la.task_key) la.task_key[la.task_seg[j] + idx] = (uint32_t)min(ip, (int64_t)UINT32_MAX);
-}
-
 __device__ void plan_no_frontier(const LongArgs& la, int row, int a0, const int64_t* ipr, int L, int H, int J,
                                  WsBase wsb, int64_t slb, int64_t tabb, int64_t chb, int64_t root_at, int y0, int dy,
                                  int64_t final_off, int* err) {
