@@ -262,7 +262,14 @@ __device__ __forceinline__ ShortMerged short_merge(int col, int p, double val, b
     const int pcol = dpp_mov<0x138, 0xF>(col, 0);  // wave_shr:1
     const int ppos = dpp_mov<0x138, 0xF>(pos, 0);
     const bool joins = alive && gl > 0 && pcol == col;
-    int lvl = joins ? 31 - __clz(pos ^ ppos) : -1;  // positions of one column differ
+    // Positions of one column differ, unless a row of B has a column twice or
+    // columns past N meet in the packed keys (the fused path merges beside the
+    // check of B).  The 1 then gives level 0, so that every entry that joins has
+    // a level from 0 to 31 and the loop below ends whatever the operands are; its
+    // indexes are lanes of the group all the same, and the product is refused.
+    // (A bound on the loop instead takes five scalar instructions a level; here
+    // the compiler drops the minimum that __clz needs for 0.)
+    int lvl = joins ? 31 - __clz((pos ^ ppos) | 1) : -1;
     asm volatile("" : "+v"(lvl));  // compared as it is, not by its parts
     uint64_t am = __ballot(alive), todo = __ballot(joins);
     for (int l = 0; todo != 0ull; ++l) {
