@@ -15,9 +15,9 @@
 //      (short_merge.h).  Every workgroup publishes its nnz, one wavefront of
 //      the grid scans these as they come and publishes each workgroup's place,
 //      and every row is written straight from registers into C, with C's row
-//      pointer.  Workgroups past the row workgroups check all of B, one B row
-//      per thread (row pointers, column range, sorted rows), as the general
-//      validation does.
+//      pointer.  Workgroups past the row workgroups check all of B, a B row
+//      per thread at a time (row pointers, column range, sorted rows), as the
+//      general validation does.
 // C is allocated beforehand for G entries per row, a bound of nnz(C) when
 // every row is short.  The scanning wavefront writes the totals and flags to
 // host memory, read once the stream has ended: a row with more than G lists or
@@ -60,9 +60,10 @@ __device__ __forceinline__ void sc_store(uint64_t* p, uint64_t v) {
 // points and an aggregation took 272 us, with the scanner 210, without any
 // wait 180.)
 // Workgroups start about in the order of their index, but nothing promises
-// it, so both waits are bounded: after SC_POLLS looks without a new word the
-// scanner marks the rest late, and the product is left to the general
-// pipeline.
+// it, so both waits are bounded: after SC_POLLS looks without a new word of a
+// row workgroup the scanner marks the rest late, and the product is left to the
+// general pipeline.  The others' words come without any bound on the looks:
+// these workgroups wait for nothing, and by then nobody waits for them.
 // nrow words of row workgroups, then those of the others.
 __device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nrow, int n, SmallResult* res) {
     const int lane = lane_id();
@@ -74,7 +75,7 @@ __device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nrow, in
         const uint64_t gap = __ballot((v & SC_SET) == 0 || base + lane >= n);
         const int got = gap ? __ffsll((long long)gap) - 1 : BRM_WAVE;  // words up to the first unpublished one
         if (got == 0) {
-            if (++polls <= SC_POLLS) continue;
+            if (base >= nrow || ++polls <= SC_POLLS) continue;
             for (int q = base + lane; q < nrow; q += BRM_WAVE) sc_store(&pre[q], SC_SET | SC_LATE);
             flags |= SC_MISS;
             break;
@@ -164,11 +165,15 @@ __global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int
     __shared__ unsigned fl[S::WPB];
     const int b = (int)blockIdx.x - 1;
     if (b >= row_blocks) {
-        // ---- B: one row per thread; entries 8 at a time (indices clamped
-        // into the row, so that every load is in bounds)
-        const int r = (b - row_blocks) * S::NT + (int)threadIdx.x;
+        // ---- B: a row per thread at a time; entries 8 at a time (indices
+        // clamped into the row, so that every load is in bounds)
+        const int64_t step = (int64_t)(words - row_blocks) * S::NT;
         bool bad = false, lng = false;
-        if (r < a.K) {
+        for (int64_t r = (int64_t)(b - row_blocks) * S::NT + threadIdx.x; r <= a.K; r += step) {
+            if (r == a.K) {
+                bad |= a.brpt[0] != 0 || a.brpt[a.K] != nnzB || a.arpt[0] != 0 || a.arpt[a.M] != nnzA;
+                continue;
+            }
             const int b0 = a.brpt[r], b1 = a.brpt[r + 1];
             if (b0 < 0 || b0 > b1 || b1 > nnzB) {
                 bad = true;
@@ -189,8 +194,6 @@ __global__ __launch_bounds__((SmallShape<G, P>::NT)) void k_small(RowArgs a, int
                     }
                 }
             }
-        } else if (r == a.K) {
-            bad = a.brpt[0] != 0 || a.brpt[a.K] != nnzB || a.arpt[0] != 0 || a.arpt[a.M] != nnzA;
         }
         const unsigned f = block_flags<S::WPB>(bad, lng, fl);
         if (threadIdx.x == 0) sc_store(&own[b], SC_SET | (uint64_t)f << SC_FLAGS);
@@ -330,11 +333,15 @@ int64_t row_blocks_of(int M) {
     return ((int64_t)M + SmallShape<G, P>::ROWS - 1) / SmallShape<G, P>::ROWS;
 }
 
-// the K rows of B and the ends of the row pointers
+// Workgroups for the K rows of B and the ends of the row pointers: SM_BMAX at
+// most, each of which takes rows in turn, as the scanner looks at every one's
+// word.  2,048 rows of 8 products, B of 2e7 rows of 2 entries: 326 us with
+// a workgroup per 512 rows (the scanner alone goes through 39,063 words), now 110.
+constexpr int SM_BMAX = 2048;
 template <int G>
 int64_t b_blocks_of(int K) {
     constexpr int NT = SmallShape<G, 1>::NT;
-    return ((int64_t)K + 1 + NT - 1) / NT;
+    return std::min(((int64_t)K + 1 + NT - 1) / NT, (int64_t)SM_BMAX);
 }
 
 template <int G, int P>
