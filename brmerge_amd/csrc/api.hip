@@ -31,7 +31,7 @@
 namespace brm {
 
 Params& params() {
-    static Params p{0, MED_CAP, 0, MED_CAP, 0, 0, GROUP_CFG_BITMAP, -1, 0, 1, 0, (int64_t)1 << 30, 0, 1, 1, 1, 1, 1};
+    static Params p{0, MED_CAP, 0, MED_CAP, 0, 0, GROUP_CFG_BITMAP, -1, 0, 1, 0, (int64_t)1 << 30, 0, 1, 1, 1, 1, 1, SMALL_LOOKS};
     return p;
 }
 
@@ -1164,10 +1164,11 @@ namespace {
 // (32 or 64) lists and products: one fill, one kernel and one host round trip
 // (small.hip).  C is allocated for `group` entries per row (a bound of nnz(C)
 // when every row is short), so nothing waits on the device before the end.
-// *handled = false when a row is longer (nothing is kept).
+// *handled = false when a row is longer, or *late, when a wait in the kernel was
+// given up (nothing is kept).
 int run_small_g(const DevIn& in, int group, int64_t max_nnz, hipStream_t s, PhaseClock& clk, DevOut* out,
-                bool* handled) {
-    *handled = false;
+                bool* handled, bool* late) {
+    *handled = *late = false;
     const int M = in.M;
     const int64_t cap = (int64_t)M * group;
     if (cap > max_nnz) return BRM_OK;
@@ -1198,8 +1199,9 @@ int run_small_g(const DevIn& in, int group, int64_t max_nnz, hipStream_t s, Phas
     HIPC(launch_small(a, in.nnzA, in.nnzB, crpt, ccol, cval, res, reinterpret_cast<uint64_t*>(words), group, s));
     HIPC(hipStreamSynchronize(s));
     const SmallResult h = *res;
-    if (h.bad) return dev_err_status(DERR_INVALID, "validation");
-    if (!h.done || h.miss || h.late) return BRM_OK;
+    if (h.flags & SMALL_BAD) return dev_err_status(DERR_INVALID, "validation");
+    *late = !h.done || h.late || (h.flags & SMALL_LATE);
+    if (*late || h.flags) return BRM_OK;
     const int64_t nnz = h.nnz, ipt = h.ip;
     sc.release(crpt);
     sc.release(ccol);
@@ -1217,17 +1219,19 @@ int run_small_g(const DevIn& in, int group, int64_t max_nnz, hipStream_t s, Phas
 }
 
 // Groups of 32 lanes (two rows per wavefront) when the average row has at
-// most 32 products, else 64; a row too long for 32 lanes retries at 64.
+// most 32 products, else 64; a row too long for 32 lanes retries at 64.  What
+// was late is not tried again.
 int run_small(const DevIn& in, double avg_ip, int64_t max_nnz, hipStream_t s, PhaseClock& clk, DevOut* out,
               bool* handled) {
     *handled = false;
     if (in.nnzA > INT32_MAX || in.nnzB > INT32_MAX) return BRM_OK;
     if (in.M < 1 || in.K < 1 || in.nnzA < 1 || in.nnzB < 1) return BRM_OK;  // C is empty: the general pipeline
+    bool late = false;
     if (avg_ip <= 32.0) {
-        BRMC(run_small_g(in, 32, max_nnz, s, clk, out, handled));
-        if (*handled) return BRM_OK;
+        BRMC(run_small_g(in, 32, max_nnz, s, clk, out, handled, &late));
+        if (*handled || late) return BRM_OK;
     }
-    return run_small_g(in, 64, max_nnz, s, clk, out, handled);
+    return run_small_g(in, 64, max_nnz, s, clk, out, handled, &late);
 }
 }  // namespace
 
@@ -1705,6 +1709,7 @@ int brm_set_param(const char* name, int64_t value) {
     else if (!strcmp(name, "cbar_budget_bytes")) { if (value < 0) return BRM_E_INVALID; p.cbar_budget_bytes = value; }
     else if (!strcmp(name, "upper_vm")) { p.upper_vm = value ? 1 : 0; }
     else if (!strcmp(name, "small_fused")) { p.small_fused = value ? 1 : 0; }
+    else if (!strcmp(name, "small_looks")) { if (value < 0 || value > SMALL_LOOKS_MAX) return BRM_E_INVALID; p.small_looks = (int)value; }
     else if (!strcmp(name, "wmed_count")) { p.wmed_count = value ? 1 : 0; }
     else if (!strcmp(name, "wmed_bitmap")) { p.wmed_bitmap = value ? 1 : 0; }
     else if (!strcmp(name, "long_tiles")) {
@@ -1735,6 +1740,7 @@ int64_t brm_get_param(const char* name) {
     if (!strcmp(name, "hash_cap")) return p.hash_cap;
     if (!strcmp(name, "upper_vm")) return p.upper_vm;
     if (!strcmp(name, "small_fused")) return p.small_fused;
+    if (!strcmp(name, "small_looks")) return p.small_looks;
     if (!strcmp(name, "wmed_count")) return p.wmed_count;
     if (!strcmp(name, "wmed_bitmap")) return p.wmed_bitmap;
     if (!strcmp(name, "long_tiles")) return p.long_tiles;

@@ -207,11 +207,13 @@ struct Params {
     int64_t sym_chunk_products; // long-row symbolic: products per list chunk (1 .. 2^30, default 2^30)
     int hash_cap;              // rows of at most hash_cap products take the hash tier (0 = off, <= HASH_CAP)
     int upper_vm;              // Upper waves grow C in reserved address ranges (1) or copy chunks (0)
-    int small_fused;           // products of few short rows in three launches (1) or the general pipeline (0)
+    int small_fused;           // products of few short rows in one kernel (1) or the general pipeline (0)
     int wmed_count;            // wavefront tier symbolic: 1 column bitmaps, 0 hash
     int wmed_bitmap;           // register tier numeric: 1 bitmap ranks (rows > 128 products), 0 sort
     int long_tiles;            // long rows: 1 the column-tile engine where its tables pay, 0 never, n >= 2 n blocks
+    int small_looks;           // fused short rows: looks without news until the scanner gives up (0 .. SMALL_LOOKS_MAX)
 };
+constexpr int SMALL_LOOKS = 1 << 14, SMALL_LOOKS_MAX = 1 << 20;
 
 // Shapes of the LDS tree-merge kernels, selectable at run time.
 struct LdsShape {

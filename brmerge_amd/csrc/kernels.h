@@ -93,19 +93,22 @@ int rmed_auto_cap(int N);
 
 // small.hip: products of at most SMALL_MAX_ROWS rows, all in the short tier.
 constexpr int SMALL_MAX_ROWS = 1 << 20;
+// Malformed operands; a row (of B: entries) too long for groups of G lanes; the
+// scanner gave up.  With any of them nothing of C is usable.
+constexpr unsigned SMALL_BAD = 1u, SMALL_MISS = 2u, SMALL_LATE = 4u;
 // What k_small tells the host, in host memory that the device can write.
 struct SmallResult {
     int done;     // the fields below are set
-    int bad;      // malformed operands
-    int miss;     // a row has more than G lists or products: nothing of C is usable
+    int flags;    // SMALL_BAD .. SMALL_LATE
     int late;     // a workgroup did not learn its place: nothing of C is usable
+    int pad;
     int64_t nnz;  // nnz(C)
     int64_t ip;   // intermediate products
 };
 // Device words (int64) for A of M and B of K rows in groups of `group` (32 or
 // 64) lanes.
 int64_t small_words(int M, int K, int group);
-// Clears the words, then merges every row and writes C's row pointer and C
+// Fills the words, then merges every row and writes C's row pointer and C
 // (capacity group * M entries).  *res is zero on entry.
 hipError_t launch_small(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
                         SmallResult* res, uint64_t* words, int group, hipStream_t s);

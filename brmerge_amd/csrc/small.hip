@@ -3,7 +3,7 @@
 // A product whose rows are all short (at most G = 64, or 32, lists and
 // products) spends more on the general pipeline's dozen launches and two
 // host round trips than on its kernels.  Such a product runs as:
-//   1. one fill clearing the words through which the workgroups' places in C
+//   1. one fill of the words through which the workgroups' places in C
 //      are handed on;
 //   2. k_small<G, P>: each workgroup takes a run of consecutive rows, in P
 //      passes of one row per group of G lanes.  The passes are batched stage
@@ -35,15 +35,13 @@ namespace brm {
 namespace {
 
 // One word per workgroup for what it adds (own) and, per row workgroup, one
-// for what comes before it (pre); cleared beforehand.  The top bit marks a
-// word as published; below it the flags, products (from bit SC_IP) and nnz(C).
+// for what comes before it (pre).  The top bit marks a word as published; below
+// it the flags (SMALL_BAD, SMALL_MISS), products (from bit SC_IP) and nnz(C).
 // Each word carries its own value, so relaxed atomics (no cache invalidation
 // or write-back) are enough.
 constexpr int SC_IP = 28, SC_FLAGS = 2 * SC_IP;
 constexpr uint64_t SC_SET = 1ull << 63, SC_LATE = 1ull << 62, SC_VAL = (1ull << SC_FLAGS) - 1ull;
-constexpr unsigned SC_BAD = 1u, SC_MISS = 2u;  // malformed operands; a row too long for this path
 static_assert((int64_t)SMALL_MAX_ROWS * BRM_WAVE < ((int64_t)1 << SC_IP), "two counts in a word");
-constexpr int SC_POLLS = 1 << 14;
 
 __device__ __forceinline__ uint64_t sc_load(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -60,31 +58,35 @@ __device__ __forceinline__ void sc_store(uint64_t* p, uint64_t v) {
 // points and an aggregation took 272 us, with the scanner 210, without any
 // wait 180.)
 // Workgroups start about in the order of their index, but nothing promises
-// it, so both waits are bounded: after SC_POLLS looks without a new word of a
-// row workgroup the scanner marks the rest late, and the product is left to the
-// general pipeline.  The others' words come without any bound on the looks:
+// it, so both waits are bounded: after more looks without a new word of a row
+// workgroup than an unpublished word says (the knob small_looks, which the host
+// fills the words with) the scanner marks the rest late, and the product is left
+// to the general pipeline.  (As an argument of the kernel the number makes the
+// row workgroups of <64, 2> take 82 scalar registers instead of 80: one of them
+// fits a CU then instead of two, and 16,384 rows of 64 products take 18.5 us
+// instead of 14.3.)  The others' words come without any bound on the looks:
 // these workgroups wait for nothing, and by then nobody waits for them.
 // nrow words of row workgroups, then those of the others.
 __device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nrow, int n, SmallResult* res) {
     const int lane = lane_id();
     uint64_t sum = 0;
     unsigned flags = 0;
-    int polls = 0;
+    int looks = 0;  // without a new word
     for (int base = 0; base < n;) {
         const uint64_t v = sc_load(&own[min(base + lane, n - 1)]);
         const uint64_t gap = __ballot((v & SC_SET) == 0 || base + lane >= n);
         const int got = gap ? __ffsll((long long)gap) - 1 : BRM_WAVE;  // words up to the first unpublished one
         if (got == 0) {
-            if (base >= nrow || ++polls <= SC_POLLS) continue;
+            if (base >= nrow || ++looks <= __builtin_amdgcn_readfirstlane((int)v)) continue;
             for (int q = base + lane; q < nrow; q += BRM_WAVE) sc_store(&pre[q], SC_SET | SC_LATE);
-            flags |= SC_MISS;
+            flags |= SMALL_LATE;
             break;
         }
-        polls = 0;
+        looks = 0;
         const uint64_t mine = lane < got ? v & SC_VAL : 0;
         const unsigned f = lane < got ? (unsigned)(v >> SC_FLAGS) : 0u;
-        if (__ballot(f & SC_BAD)) flags |= SC_BAD;
-        if (__ballot(f & SC_MISS)) flags |= SC_MISS;
+        if (__ballot(f & SMALL_BAD)) flags |= SMALL_BAD;
+        if (__ballot(f & SMALL_MISS)) flags |= SMALL_MISS;
         const uint64_t inc = wave_incl_scan(mine);
         if (lane < got && base + lane < nrow) sc_store(&pre[base + lane], SC_SET | (sum + inc - mine));
         sum += wave_last(inc);
@@ -93,8 +95,7 @@ __device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nrow, in
     if (lane == 0) {
         res->nnz = (int64_t)(sum & ((1ull << SC_IP) - 1ull));
         res->ip = (int64_t)(sum >> SC_IP);
-        res->bad = (flags & SC_BAD) != 0;
-        res->miss = (flags & SC_MISS) != 0;
+        res->flags = (int)flags;
         res->done = 1;
     }
 }
@@ -103,7 +104,7 @@ __device__ void scan_workgroups(const uint64_t* own, uint64_t* pre, int nrow, in
 // wavefront).
 template <int NW>
 __device__ unsigned block_flags(bool bad, bool miss, unsigned* fl) {
-    const unsigned mine = (__ballot(bad) != 0ull ? SC_BAD : 0u) | (__ballot(miss) != 0ull ? SC_MISS : 0u);
+    const unsigned mine = (__ballot(bad) != 0ull ? SMALL_BAD : 0u) | (__ballot(miss) != 0ull ? SMALL_MISS : 0u);
     if (lane_id() == 0) fl[threadIdx.x / BRM_WAVE] = mine;
     __syncthreads();
     unsigned f = 0u;
@@ -115,7 +116,7 @@ __device__ unsigned block_flags(bool bad, bool miss, unsigned* fl) {
 // The prefix of workgroup b (called by one wavefront); 0 and *late when it
 // does not come.
 __device__ uint64_t await_prefix(const uint64_t* pre, int b, bool* late) {
-    for (int polls = 0; polls < 4 * SC_POLLS; ++polls) {
+    for (int looks = 0; looks < 4 * SMALL_LOOKS; ++looks) {
         const uint64_t v = sc_load(&pre[b]);
         if (v & SC_SET) {
             *late = (v & SC_LATE) != 0;
@@ -393,7 +394,7 @@ int64_t small_words(int M, int K, int group) { return group == 32 ? words_of<32>
 hipError_t launch_small(const RowArgs& a, int64_t nnzA, int64_t nnzB, int64_t* crpt, int* ccol, double* cval,
                         SmallResult* res, uint64_t* words, int group, hipStream_t s) {
     if (a.M < 1 || a.K < 1 || nnzA < 1 || nnzB < 1) return hipErrorInvalidValue;
-    hipError_t e = launch_fill_i64((int64_t*)words, small_words(a.M, a.K, group), 0, s);
+    hipError_t e = launch_fill_i64((int64_t*)words, small_words(a.M, a.K, group), params().small_looks, s);
     if (e != hipSuccess) return e;
     return group == 32 ? launch_small_g<32>(a, nnzA, nnzB, crpt, ccol, cval, res, words, s)
                        : launch_small_g<64>(a, nnzA, nnzB, crpt, ccol, cval, res, words, s);

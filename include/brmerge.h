@@ -158,7 +158,7 @@ int brm_flop_count_dev(const int *arpt, const int *acol, int64_t nnzA, const int
  * "force_long", "profile", "lds_cfg", "group_cfg", "wmed_cap",
  * "wmed_engine", "launch_chunk", "cbar_budget_bytes", "sym_chunk_products",
  * "hash_cap", "upper_vm", "small_fused", "wmed_count", "wmed_bitmap",
- * "long_tiles");
+ * "long_tiles", "small_looks");
  * returns BRM_E_INVALID for unknown names or
  * values.  Knobs other than hash_cap never change results, only speed.  group_cfg 0-3:
  * merge-path engine shapes for long rows; 4 (default): the bitmap-rank
@@ -178,7 +178,9 @@ int brm_flop_count_dev(const int *arpt, const int *acol, int64_t nnzA, const int
  * BRMerge-Upper's row waves compact into C grown in a reserved address range;
  * 0 (or a driver without address reservation): into chunks copied into C.
  * small_fused (1, the default): products whose rows are all short run in
- * the three-launch fused path.  wmed_count (1, the default): the
+ * one fused kernel.  small_looks (16,384, at most 2^20): how often that
+ * kernel looks in vain for its workgroups' counts before it leaves the
+ * product to the general pipeline.  wmed_count (1, the default): the
  * wavefront tier's row lengths are counted with column bitmaps; 0: with the
  * hash count.  wmed_bitmap (1, the default): the register tier ranks rows of
  * more than 128 products with column bitmaps (and takes rows of up to 2,048
