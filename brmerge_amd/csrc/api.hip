@@ -334,9 +334,9 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         last = budget;
     }
     // The column-tile engine where its tables pay: block boundaries and B's
-    // table rows, at most a quarter of the budget and taken off it.  Not in
-    // the fixed-buffer arena; and where they cannot be allocated the engine
-    // without tables runs.
+    // table rows, at most a quarter of the budget and taken off it, and the
+    // waves' node tables, counted to their rows.  Not in the fixed-buffer arena;
+    // and where any of them cannot be allocated the engine without tables runs.
     Scratch tile_sc;
     int nb = 0;
     int *tile_cb = nullptr, *tile_brow = nullptr;
@@ -377,8 +377,9 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
         return n;
     };
     std::vector<int64_t> rbytes(nlong);
+    const int tab_sets = thread_side_streams() ? 2 : 1;  // waves that overlap have a node table each
     for (int k = 0; k < nlong; ++k)
-        rbytes[k] = 4 * (int64_t)(nb + 1) * n_nodes(k) + 12 * (ws_need(k, 0) + ws_need(k, 1)) + 8 * ((int64_t)2 << hk[k]) +
+        rbytes[k] = 4 * (int64_t)(nb + 1) * n_nodes(k) * tab_sets + 12 * (ws_need(k, 0) + ws_need(k, 1)) + 8 * ((int64_t)2 << hk[k]) +
                     (int64_t)(sizeof(GroupTask) + sizeof(LeafTask) + 2 * sizeof(Child)) * (len[k] + 16);
 
     tr.mark("long info read back");
@@ -498,7 +499,8 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
     // not hold the sort's buffers).
     struct WaveTables {
         int* rows_w = nullptr;
-        int64_t *wsb_d = nullptr, *slb_d = nullptr, *tabb_d = nullptr, *chb_d = nullptr, *root_d = nullptr, *seg_d = nullptr, *slots = nullptr, *counters = nullptr;
+        int64_t *wsb_d = nullptr, *slb_d = nullptr, *tabb_d = nullptr, *chb_d = nullptr, *root_d = nullptr;
+        int64_t *seg_d = nullptr, *slots = nullptr, *counters = nullptr;
         GroupTask* tasks = nullptr;
         Child* children = nullptr;
         int *node_tab = nullptr, *large_d = nullptr;
@@ -527,10 +529,6 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
             BRMC(wsc.alloc(&t.root_d, mx_rows, "wave root_task"));
             BRMC(wsc.alloc(&t.large_d, mx_rows, "wave large rows"));
         }
-        if (nb > 0) {
-            BRMC(wsc.alloc(&t.tabb_d, mx_rows, "wave tab_base"));
-            BRMC(wsc.alloc(&t.node_tab, mx_tab, "node block table"));
-        }
         BRMC(wsc.alloc(&t.seg_d, MAX_PASSES + 2, "task segments"));
         BRMC(wsc.alloc(&t.slots, mx_sl, "length slots"));
         BRMC(wsc.alloc(&t.counters, CNT_N, "planner counters"));
@@ -543,6 +541,20 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
             BRMC(wsc.alloc(&t.tidx_out, mx_task, "task order"));
             BRMC(wsc.alloc(&t.ttmp, (int64_t)ttmp_bytes, "task sort"));
         }
+    }
+    // node tables last, when all that the engine without them needs is there
+    for (int par = 0; par < (overlap ? 2 : 1) && nb > 0; ++par) {
+        WaveTables& t = wt[par];
+        if (wsc.alloc(&t.tabb_d, mx_rows, "wave tab_base") == BRM_OK &&
+            wsc.alloc(&t.node_tab, mx_tab, "node block table") == BRM_OK)
+            continue;
+        for (WaveTables& u : wt) {
+            if (u.tabb_d) wsc.free_now(u.tabb_d);
+            if (u.node_tab) wsc.free_now(u.node_tab);
+            u.tabb_d = nullptr;
+            u.node_tab = nullptr;
+        }
+        nb = 0;
     }
     tr.mark("workspace allocated", mx_ws[0] + mx_ws[1]);
     int* const wcol[2] = {wcol0, wcol1};
