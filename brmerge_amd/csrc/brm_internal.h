@@ -267,6 +267,5 @@ struct ProfScope {
 // Product count of each A entry (|B row acol[j]|, 0 for a column outside [0, K)).
 hipError_t scan_alen(const int* acol, const int* brpt, int K, int64_t n, int64_t* out, hipStream_t s);
 hipError_t scan_i64(const int64_t* in, int64_t n, int64_t* out, hipStream_t s);
-hipError_t scan_i32(const int* in, int64_t n, int64_t* out, hipStream_t s);
 
 }  // namespace brm

@@ -79,16 +79,17 @@ hipError_t order_rows(int* rows, int n, const int* arpt, const int64_t* ipA, uin
 hipError_t order_tasks(const uint32_t* keys, int n, uint32_t* keys_out, int* idx_in, int* idx_out, void* tmp,
                        size_t tmp_bytes, hipStream_t s);
 
-// rmed.hip (register tier; cap = products per row, <= WMED_CAP)
+// rmed.hip (register tier; cap = products per row, <= WMED_CAP_BITMAP)
 hipError_t launch_rmed_numeric(const int* rows, int n, const RowArgs& a, const OutArgs& o, hipStream_t s, int cap);
 // Exact row lengths of register-tier rows (ip <= cap, at most 64 lists) by
 // LDS column bitmaps.
-// Largest register-tier row (products) for B of N columns under the current
-// knobs: WMED_CAP_BITMAP where the bitmap ranks apply, else WMED_CAP.
-int rmed_max_cap(int N);
 hipError_t launch_rmed_count(const int* rows, int n, const RowArgs& a, int64_t* nnzrow, hipStream_t s, int cap);
-// Wavefront-tier capacity chosen when wmed_cap is -1 (register engine): 1024
-// products while 32-bit sort keys hold N columns, else 512.
+// Largest register-tier row (products) for B of N columns under the current
+// knobs: WMED_CAP_BITMAP with bitmap ranks and at most 2^20 columns, else
+// WMED_CAP.
+int rmed_max_cap(int N);
+// The same when wmed_cap is -1 (register engine): WMED_CAP_BITMAP likewise,
+// else 1024 products for at most 2^16 columns, else 512.
 int rmed_auto_cap(int N);
 
 // small.hip: products of at most SMALL_MAX_ROWS rows, all in the short tier.

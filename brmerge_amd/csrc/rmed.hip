@@ -94,7 +94,7 @@ static_assert(sizeof(RmLists) <= sizeof(RmSmem<2, uint32_t>), "list table fits t
 //
 // Ranks come in levels of 64-way fan-out.  The top level has one bit per
 // 2^SH columns of the row's own column span, SH the least of 0, 6, 12, 18
-// for which the span fits RB_NW words of 64 bits; each level below holds one
+// for which the span fits rb_words<R>() words of 64 bits; each level below holds one
 // 64-bit word per bit set above it (at most one per product), so its words
 // are numbered by the popcount ranks of the level above, and the ranks of
 // the last level (SH = 0) are the output positions.  A banded row takes one
@@ -422,7 +422,7 @@ __device__ __forceinline__ void rmed_outputs(const int (&col)[R], const int (&lp
         if (pairs) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                    if (lane < ip - r * 64 && pos[r] >= 0x10000) {
+                if (lane < ip - r * 64 && pos[r] >= 0x10000) {
                     const int q = pos[r] & 0xffff;
                     const double x = B.val[q];
                     B.val[q] = (int)B.lp[q] < lp[r] ? fadd(x, prod[r]) : fadd(prod[r], x);
@@ -823,9 +823,12 @@ constexpr int RM_WIDE = 1 << 20;
 int rmed_auto_cap(int N) {
     // With bitmap ranks rows of up to WMED_CAP_BITMAP products while B has at
     // most RM_WIDE columns (rows of 1025-2048 products: 2,048 products per
-    // wavefront ran faster than the workgroup LDS tier).  Otherwise 1024
-    // products while 32-bit sort keys hold N columns beside 16 bits of
-    // position and index, else 512.
+    // wavefront ran faster than the workgroup LDS tier).  Otherwise the sort's
+    // limits: 1024 products while 32-bit keys hold N columns beside 16 bits of
+    // position and index, else 512.  Above RM_WIDE columns that is not the
+    // ranks' own limit, which serve any N: the rows between run faster with
+    // wmed_cap 1024 than in the LDS tier (200,000 rows of 600 products, 1.5e6
+    // columns: 1.09 ms against 19.0; 120,000 of 990: 0.97 against 15.9).
     if (params().wmed_bitmap == 1 && N <= RM_WIDE) return WMED_CAP_BITMAP;
     return (int64_t)N - 1 <= RmKey<16, uint32_t>::COL_MAX ? 1024 : 512;
 }

@@ -50,14 +50,13 @@ struct AlenF {
     }
 };
 // Array elements.
-template <typename S>
 struct ArrayF {
     static constexpr bool STASH = false;
-    const S* p;
+    const int64_t* p;
     template <int N, typename T>
     __device__ void load(const int64_t (&j)[N], int64_t n, T (&x)[N]) const {
 #pragma unroll
-        for (int i = 0; i < N; ++i) x[i] = j[i] < n ? (T)p[j[i]] : (T)0;
+        for (int i = 0; i < N; ++i) x[i] = j[i] < n ? p[j[i]] : 0;
     }
 };
 // Element i of this thread's share of the tile at base.
@@ -134,7 +133,7 @@ __global__ __launch_bounds__(SCAN_PNT) void k_scan_partials(int64_t* part, int64
     constexpr int ITEMS = 8;
     int64_t carry = 0;
     for (int64_t base = 0; base < nb; base += SCAN_PNT * ITEMS) {
-        carry += scan_tile<SCAN_PNT, ArrayF<int64_t>, ITEMS>(ArrayF<int64_t>{part}, nb, base, carry, part, sm);
+        carry += scan_tile<SCAN_PNT, ArrayF, ITEMS>(ArrayF{part}, nb, base, carry, part, sm);
         __syncthreads();  // sm is written again
     }
     if (threadIdx.x == 0) part[nb] = carry;
@@ -213,10 +212,7 @@ hipError_t scan_alen(const int* acol, const int* brpt, int K, int64_t n, int64_t
     return scan(AlenF{acol, brpt, K}, n, out, s);
 }
 hipError_t scan_i64(const int64_t* in, int64_t n, int64_t* out, hipStream_t s) {
-    return scan(ArrayF<int64_t>{in}, n, out, s);
-}
-hipError_t scan_i32(const int* in, int64_t n, int64_t* out, hipStream_t s) {
-    return scan(ArrayF<int>{in}, n, out, s);
+    return scan(ArrayF{in}, n, out, s);
 }
 
 }  // namespace brm
