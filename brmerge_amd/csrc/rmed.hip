@@ -111,8 +111,9 @@ static_assert(sizeof(RmLists) <= sizeof(RmSmem<2, uint32_t>), "list table fits t
 // products, N = 1.5e6: 4.04 -> 1.68 ms, and their count 1.07 (hash) -> 0.82.
 // Then, several rows per wavefront (rm_rows), products without lanes of
 // their own as repeats of the last one, and as many registers as the row
-// needs (rm_step): 3.01 -> 2.29 ms and 685 instructions, count 0.82 -> 0.62 ms.
-// The LDS pipe is now busy most of the time, the VALU three quarters of it.
+// needs (rm_step): 3.01 -> 2.32 ms and 750 instructions, count 0.82 -> 0.62 ms.
+// The vector units are then busy 0.68 of the time (0.74 at R = 4), and bank
+// conflicts take a fifth of the LDS cycles.
 template <int R>
 constexpr int rb_words() {
     return R < 4 ? 256 : 64 * R;  // words of one level: at least one per product
