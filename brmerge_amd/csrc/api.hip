@@ -31,7 +31,8 @@
 namespace brm {
 
 Params& params() {
-    static Params p{0, MED_CAP, 0, MED_CAP, 0, 0, GROUP_CFG_BITMAP, -1, 0, 1, 0, (int64_t)1 << 30, 0, 1, 1, 1, 1, 1, SMALL_LOOKS};
+    static Params p{0, MED_CAP, 0, MED_CAP, 0, 0, GROUP_CFG_BITMAP, -1, 0, 1, 0, (int64_t)1 << 30,
+                    0, 1, 1, 1, 1, 1, SMALL_LOOKS};
     return p;
 }
 
@@ -379,7 +380,8 @@ int run_long(const RowArgs& a, const int* rows_d, int nlong, const OutArgs& o, c
     std::vector<int64_t> rbytes(nlong);
     const int tab_sets = thread_side_streams() ? 2 : 1;  // waves that overlap have a node table each
     for (int k = 0; k < nlong; ++k)
-        rbytes[k] = 4 * (int64_t)(nb + 1) * n_nodes(k) * tab_sets + 12 * (ws_need(k, 0) + ws_need(k, 1)) + 8 * ((int64_t)2 << hk[k]) +
+        rbytes[k] = 4 * (int64_t)(nb + 1) * n_nodes(k) * tab_sets + 12 * (ws_need(k, 0) + ws_need(k, 1)) +
+                    8 * ((int64_t)2 << hk[k]) +
                     (int64_t)(sizeof(GroupTask) + sizeof(LeafTask) + 2 * sizeof(Child)) * (len[k] + 16);
 
     tr.mark("long info read back");
